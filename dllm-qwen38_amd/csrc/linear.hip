@@ -25,7 +25,10 @@
 //     between workgroups leaves an fp32 partial per piece (at most two per workgroup: its first
 //     and its last piece); a second kernel sums the pieces in workgroup order (deterministic) for
 //     the split tiles only;
-//   * more than 32 token rows: the next 32 rows are further tiles (the weights are streamed again);
+//   * more than 32 token rows (two sequences' blocks): tiles of 64 rows, so that the weights are
+//     still streamed once; a unit then stages 24 KB and each wave issues eight MFMAs. With 32-row
+//     tiles the second 32 rows streamed every weight again (MLP of hidden 5120 and width 17408 at 64
+//     rows, 0.54 GB of weights: 205.3 -> 127.0 us, 2.6 -> 4.3 TB/s);
 //   * up to four projections of the same x (q | k | v, the four mixer inputs, gate | up) share one
 //     launch: the feature tiles run through the weights in turn. With the SwiGLU epilogue
 //     (gate | up) the second kernel writes round(round(silu(gate)) * up), the MLP's activation,
@@ -42,11 +45,10 @@
 
 namespace dllm {
 
-constexpr int LIN_NST = 4;                 // ring stages (4 x 20 KB: two workgroups fit a CU)
+constexpr int LIN_NST = 4;                 // ring stages (4 x 20 KB with 32 rows: two workgroups fit a CU)
 constexpr int LIN_W_BYTES = 128 * 64 * 2;  // weight tile of one unit
-constexpr int LIN_X_BYTES = 32 * 64 * 2;   // token tile of one unit
-constexpr int LIN_STAGE = LIN_W_BYTES + LIN_X_BYTES;
-constexpr int LIN_TILE = 32 * 128;         // floats of one partial tile
+constexpr int LIN_X_BYTES = 32 * 64 * 2;   // 32 token rows of one unit
+constexpr int LIN_TILE = 32 * 128;         // floats of 32 rows of a partial tile
 constexpr int LIN_CUS = 256;               // compute units of the chip (MI355X)
 
 __device__ __forceinline__ int lin_off(int row, int chunk) {  // byte offset of a 16-byte chunk of a 128-byte row
@@ -80,12 +82,13 @@ struct LinSeg {
 struct LinArgs {
   const bf16* x;
   LinSeg seg[LIN_MAXSEG];
-  float* part;    // [G][2][32][128] fp32 partial tiles: a workgroup's first and last piece
+  float* part;    // [G][2][tr][128] fp32 partial tiles: a workgroup's first and last piece
   bf16* up;       // swiglu: the up projection's whole tiles [M, N], rounded
   int nseg, M, K;
   int ntn;        // feature tiles over all projections
   int ns;         // units per tile (K / 64)
-  int units;      // tiles * ns, tiles = ntn * ceil(M / 32)
+  int tr, pt;     // token rows per tile (32 or 64), floats of one partial tile (tr * 128)
+  int units;      // tiles * ns, tiles = ntn * ceil(M / tr)
   int uq, ur;     // units = uq * G + ur
   int G, swiglu;
 };
@@ -106,7 +109,10 @@ __device__ __forceinline__ int lin_seg(const LinArgs& a, int nt) {  // projectio
   return si;
 }
 
+// MT: 32-row groups of token rows per tile (a.tr = 32 MT)
+template <int MT>
 __global__ __launch_bounds__(256) void decode_linear_kernel(LinArgs a) {
+  constexpr int LIN_STAGE = LIN_W_BYTES + MT * LIN_X_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char smem[LIN_NST * LIN_STAGE];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -122,7 +128,7 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(LinArgs a) {
   auto stage = [&](int j) {  // unit u0 + j into ring slot j % LIN_NST
     const int mt = st_tile / a.ntn, nt = st_tile - mt * a.ntn;
     const LinSeg& sg = a.seg[lin_seg(a, nt)];
-    const int n0 = (nt - sg.tile0) * 128, m0 = mt * 32, k0 = 64 * st_step;
+    const int n0 = (nt - sg.tile0) * 128, m0 = mt * 32 * MT, k0 = 64 * st_step;
     unsigned char* sb = smem + (j % LIN_NST) * LIN_STAGE;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {  // this wave's 4 of the 16 weight instructions: rows 32 wave + 8 i ..
@@ -131,21 +137,22 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(LinArgs a) {
       const int c = schunk ^ ((row >> 1) & 7);
       dma_load16_stream(sg.w + (long long)n * K + k0 + 8 * c, sb + (32 * wave + 8 * i) * 128);
     }
-    {  // token tile: wave w stages rows 8 w .. 8 w + 7
-      const int row = 8 * wave + srow;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {  // token tile: wave w stages rows 8 w .. 8 w + 7 of each 32
+      const int row = 32 * i + 8 * wave + srow;
       const int m = min(m0 + row, M - 1);
       const int c = schunk ^ ((row >> 1) & 7);
-      dma_load16(x + (long long)m * K + k0 + 8 * c, sb + LIN_W_BYTES + 8 * wave * 128);
+      dma_load16(x + (long long)m * K + k0 + 8 * c, sb + LIN_W_BYTES + (32 * i + 8 * wave) * 128);
     }
     if (++st_step == ns) st_step = 0, ++st_tile;
   };
-  constexpr int PER = 5;  // direct loads per wave per unit
+  constexpr int PER = 4 + MT;  // direct loads per wave per unit
   static_assert(LIN_NST >= 2 && LIN_NST * LIN_STAGE <= 160 * 1024, "ring depth");
   // unit j has landed for this wave; the units issued after it may still travel
   auto wait_unit = [&](int j) { lin_wait_behind<LIN_NST - 2, PER>(min(LIN_NST - 2, nunits - 1 - j)); };
 
-  // acc: lane holds feature column l32 of this wave's 32 features, token rows rho(v, h)
-  auto flush = [&](int tile, bool whole, int slot, const f32x16& acc) {
+  // acc[i]: lane holds feature column l32 of this wave's 32 features, token rows 32 i + rho(v, h)
+  auto flush = [&](int tile, bool whole, int slot, const f32x16 (&acc)[MT]) {
     const int mt = tile / a.ntn, nt = tile - mt * a.ntn;
     const int si = lin_seg(a, nt);
     const LinSeg& sg = a.seg[si];
@@ -154,18 +161,24 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(LinArgs a) {
       bf16* const y = (a.swiglu && si == 1) ? a.up : sg.y;
       if (n >= sg.N) return;
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int m = mt * 32 + rho(v, h);
-        if (m < M) y[(long long)m * sg.N + n] = (bf16)acc[v];
-      }
-    } else {
-      float* const p = a.part + (long long)(2 * blockIdx.x + slot) * LIN_TILE + 32 * wave + l32;
+      for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) p[rho(v, h) * 128] = acc[v];
+        for (int v = 0; v < 16; ++v) {
+          const int m = (mt * MT + i) * 32 + rho(v, h);
+          if (m < M) y[(long long)m * sg.N + n] = (bf16)acc[i][v];
+        }
+    } else {
+      float* const p = a.part + (long long)(2 * blockIdx.x + slot) * (MT * LIN_TILE) + 32 * wave + l32;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) p[(32 * i + rho(v, h)) * 128] = acc[i][v];
     }
   };
 
-  f32x16 acc = zero16();
+  f32x16 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = zero16();
 #pragma unroll
   for (int j = 0; j < LIN_NST - 1; ++j)
     if (j < nunits) stage(j);
@@ -177,17 +190,22 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(LinArgs a) {
     if (j + LIN_NST - 1 < nunits) stage(j + LIN_NST - 1);  // its slot held unit j - 1, done before the barrier
     const unsigned char* sb = smem + (j % LIN_NST) * LIN_STAGE;
     const unsigned char* xs = sb + LIN_W_BYTES;
-    bf16x8 av[4], bv[4];
+    bf16x8 av[MT][4], bv[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      av[u] = *(const bf16x8*)(xs + lin_off(l32, 2 * u + h));
+#pragma unroll
+      for (int i = 0; i < MT; ++i) av[i][u] = *(const bf16x8*)(xs + lin_off(32 * i + l32, 2 * u + h));
       bv[u] = *(const bf16x8*)(sb + lin_off(32 * wave + l32, 2 * u + h));
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[u], bv[u], acc, 0, 0, 0);
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+        acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i][u], bv[u], acc[i], 0, 0, 0);
     if (step == ns - 1 || j == nunits - 1) {  // the piece ends: the tile's last unit or the range's
       flush(tile, pstep0 == 0 && step == ns - 1, slot, acc);
-      acc = zero16();
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[i] = zero16();
       slot = 1;
       pstep0 = 0;
     }
@@ -203,7 +221,7 @@ __global__ __launch_bounds__(256) void decode_linear_kernel(LinArgs a) {
 // its last, slot 1). The pieces' 16-byte loads go out eight at a time before their sums.
 __device__ __forceinline__ f32x4 lin_sum_pieces(const LinArgs& a, int t0, int w0, int w1, int q) {
   const f32x4* const p = (const f32x4*)a.part + q;
-  constexpr int T4 = LIN_TILE / 4;
+  const int T4 = a.pt / 4;
   f32x4 s = p[(long long)(2 * w0 + (lin_start(a, w0) >= t0 ? 0 : 1)) * T4];
   for (int wb = w0 + 1; wb <= w1; wb += 8) {
     f32x4 v[8];
@@ -222,7 +240,7 @@ struct LinFix {
   int n;                   // split tiles in this launch
   int tile[LIN_FIXMAX];
 };
-constexpr int LIN_FIX_CHUNKS = LIN_TILE / 4 / 256;  // blocks per tile: one float4 per thread
+constexpr int LIN_FIX_CHUNKS = LIN_TILE / 4 / 256;  // blocks per 32 rows of a tile: one float4 per thread
 
 // Tiles split between workgroups (listed by the host): block (i, c) sums chunk c of tile i's pieces.
 __global__ __launch_bounds__(256) void decode_linear_fixup_kernel(LinArgs a, LinFix f) {
@@ -232,7 +250,7 @@ __global__ __launch_bounds__(256) void decode_linear_fixup_kernel(LinArgs a, Lin
   const LinSeg& sg = a.seg[lin_seg(a, nt)];
   const int q = blockIdx.y * 256 + threadIdx.x;
   const f32x4 s = lin_sum_pieces(a, t0, w0, w1, q);
-  const int m = mt * 32 + (q >> 5), n = (nt - sg.tile0) * 128 + 4 * (q & 31);
+  const int m = mt * a.tr + (q >> 5), n = (nt - sg.tile0) * 128 + 4 * (q & 31);
   if (m >= a.M) return;
   bf16* const y = sg.y + (long long)m * sg.N;
 #pragma unroll
@@ -255,7 +273,7 @@ struct GdnPrologue {
   int width, P;        // conv width; carry-in length (0 or width - 1)
 };
 
-// One block per output tile (32 rows x 128 features): the tile's rounded values (stored whole by
+// One block per 32 rows x 128 features of the outputs: their rounded values (stored whole by
 // the streaming kernel, or its pieces summed in workgroup order and stored, as the fixup does; all
 // of a thread's loads go out before their sums) go to LDS, then by projection:
 //   qkv: the causal depthwise conv + SiLU (width KW) of every (row, channel) of the tile, as the
@@ -271,12 +289,11 @@ template <typename TW, typename TP, int KW>
 __global__ __launch_bounds__(256) void decode_gdn_prologue_kernel(LinArgs a, GdnPrologue p) {
   static_assert(KW >= 2 && KW <= 8, "conv width");
   __shared__ float vals[32][129];
-  const int tile = blockIdx.x;
-  const int mt = tile / a.ntn, nt = tile - mt * a.ntn;
+  const int mt = blockIdx.x / a.ntn, nt = blockIdx.x - mt * a.ntn;  // 32-row block, feature tile
   const int si = lin_seg(a, nt);
   const LinSeg& sg = a.seg[si];
   const int n0 = (nt - sg.tile0) * 128;
-  const int t0 = tile * a.ns;
+  const int t0 = ((mt * 32 / a.tr) * a.ntn + nt) * a.ns;
   const int w0 = lin_owner(a, t0), w1 = lin_owner(a, t0 + a.ns - 1);
   const bool split = w0 != w1;
   if (si == 1 && !split) return;
@@ -316,8 +333,8 @@ __global__ __launch_bounds__(256) void decode_gdn_prologue_kernel(LinArgs a, Gdn
   }
   constexpr int KQ = LIN_TILE / 4 / 256;  // float4 slots per thread: q = k 256 + tid, row q / 32, features 4 (q % 32) ..
   if (split) {
-    constexpr int T4 = LIN_TILE / 4;
-    const f32x4* const pp = (const f32x4*)a.part + threadIdx.x;
+    const int T4 = a.pt / 4;
+    const f32x4* const pp = (const f32x4*)a.part + (mt * 32 % a.tr) * 32 + threadIdx.x;
     const long long first = (long long)(2 * w0 + (lin_start(a, w0) >= t0 ? 0 : 1)) * T4;
     f32x4 sum[KQ];
 #pragma unroll
@@ -412,14 +429,14 @@ __global__ __launch_bounds__(256) void decode_gdn_prologue_kernel(LinArgs a, Gdn
 // up), gate and up each the rounded sum of their tile (stored whole by the main kernel, or summed
 // here from the pieces).
 __global__ __launch_bounds__(256) void decode_linear_swiglu_kernel(LinArgs a) {
-  const int ntg = a.seg[1].tile0;  // gate tiles per 32 token rows
+  const int ntg = a.seg[1].tile0;  // gate tiles per row tile
   const int mt = blockIdx.x / ntg, ng = blockIdx.x - mt * ntg;
   const int tg = mt * a.ntn + ng, tu = tg + ntg;
   const int N = a.seg[0].N;
   const int g0 = tg * a.ns, gw0 = lin_owner(a, g0), gw1 = lin_owner(a, g0 + a.ns - 1);
   const int u0 = tu * a.ns, uw0 = lin_owner(a, u0), uw1 = lin_owner(a, u0 + a.ns - 1);
   const int q = blockIdx.y * 256 + threadIdx.x;
-  const int m = mt * 32 + (q >> 5), n = ng * 128 + 4 * (q & 31);
+  const int m = mt * a.tr + (q >> 5), n = ng * 128 + 4 * (q & 31);
   if (m >= a.M) return;
   f32x4 gs = {}, us = {};
   if (gw0 != gw1) gs = lin_sum_pieces(a, g0, gw0, gw1, q);
@@ -456,7 +473,7 @@ __global__ __launch_bounds__(1024) void decode_linear_rmsnorm_kernel(LinArgs a, 
   float* const part = (float*)(lin_rms_smem + (size_t)a.seg[0].N * sizeof(bf16));  // [8]
   typedef __attribute__((ext_vector_type(8))) TW W8;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int m = blockIdx.x, mt = m >> 5, mr = m & 31;
+  const int m = blockIdx.x, mt = m / a.tr, mr = m - mt * a.tr;
   const int N = a.seg[0].N;
   const long long base = (long long)m * N;
   const bool norm_wave = wv < nw;
@@ -479,12 +496,12 @@ __global__ __launch_bounds__(1024) void decode_linear_rmsnorm_kernel(LinArgs a, 
       yv = *(const bf16x4*)(a.seg[0].y + base + c);
     } else {
       const float* const p = a.part + mr * 128 + (c & 127);
-      f32x4 sum = *(const f32x4*)(p + (long long)(2 * w0 + (lin_start(a, w0) >= t0 ? 0 : 1)) * LIN_TILE);
+      f32x4 sum = *(const f32x4*)(p + (long long)(2 * w0 + (lin_start(a, w0) >= t0 ? 0 : 1)) * a.pt);
       for (int wb = w0 + 1; wb <= w1; wb += 8) {
         f32x4 pc[8];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-          if (wb + i <= w1) pc[i] = *(const f32x4*)(p + (long long)(2 * (wb + i)) * LIN_TILE);
+          if (wb + i <= w1) pc[i] = *(const f32x4*)(p + (long long)(2 * (wb + i)) * a.pt);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           if (wb + i <= w1) sum += pc[i];
@@ -537,12 +554,24 @@ __global__ __launch_bounds__(1024) void decode_linear_rmsnorm_kernel(LinArgs a, 
 
 using namespace dllm;
 
-static long long lin_units(int M, long long ntn, int K) { return ntn * ((M + 31) / 32) * (K / 64); }
+static long long lin_units(int M, long long ntn, int K, int tr) { return ntn * ((M + tr - 1) / tr) * (K / 64); }
+
+// Token rows per tile: 64 for more than 32 rows, so that the weights are streamed once, unless more
+// than one workgroup per CU would split such tiles (pieces of twice the size in more workgroups
+// than the allocation-free array holds), where tiles stay at 32 rows. With 64-row tiles, G
+// workgroups split none when G divides the tiles (or a tile is one unit).
+static int lin_rows(int M, long long ntn, int K, long long G) {
+  if (M <= 32) return 32;
+  const long long ns = K / 64, u = ntn * ns;
+  if (G > u) G = u;
+  const bool split = ns > 1 && ntn % G != 0;
+  return split && G > LIN_CUS ? 32 : 64;
+}
 
 extern "C" int dllm_decode_linear_workgroups(int M, int N, int K) {
   if (M <= 0 || M > 64 || N <= 0 || K <= 0 || K % 64) return 0;
-  const long long tiles = (long long)((N + 127) / 128) * ((M + 31) / 32);
-  const long long u = tiles * (K / 64);
+  const long long tiles = (N + 127) / 128;
+  const long long u = tiles * ((M + 31) / 32) * (K / 64);
   if (u > 0x7fffffffLL) return 0;
   // enough whole tiles to fill the chip twice over: one tile per workgroup, nothing split;
   // otherwise one workgroup per CU, each an equal share of the units
@@ -552,7 +581,7 @@ extern "C" int dllm_decode_linear_workgroups(int M, int N, int K) {
 
 extern "C" long long dllm_decode_linear_workspace_bytes(int M, int N_gate, int workgroups, int swiglu) {
   if (M <= 0 || workgroups <= 0 || N_gate < 0) return -1;
-  long long b = (long long)workgroups * 2 * LIN_TILE * sizeof(float);
+  long long b = (long long)workgroups * 2 * LIN_TILE * (M > 32 ? 2 : 1) * sizeof(float);
   if (swiglu) b += ((long long)M * N_gate * 2 + 255) / 256 * 256;
   return b;
 }
@@ -588,17 +617,22 @@ static int lin_launch_main(const void* x, int M, int K, int count, const void* c
     sg.tile0 = (int)ntn;
     ntn += (Ns[i] + 127) / 128;
   }
-  const long long units = lin_units(M, ntn, K);
-  if (units > 0x7fffffffLL) return fail(DLLM_EUNSUPPORTED, "decode linear: %lld work units is too many", units);
+  if (lin_units(M, ntn, K, 32) > 0x7fffffffLL)
+    return fail(DLLM_EUNSUPPORTED, "decode linear: %lld work units is too many", lin_units(M, ntn, K, 32));
+  if (workgroups > 32768 && lin_units(M, ntn, K, 32) > 32768)
+    return fail(DLLM_EINVAL, "decode linear: %d workgroups (at most 32768)", workgroups);
+  a.tr = lin_rows(M, ntn, K, workgroups);
+  a.pt = a.tr * 128;
+  const long long units = lin_units(M, ntn, K, a.tr);
   a.ntn = (int)ntn;
   a.units = (int)units;
   a.G = workgroups < units ? workgroups : (int)units;  // no workgroup without units
-  if (a.G > 32768) return fail(DLLM_EINVAL, "decode linear: %d workgroups (at most 32768)", workgroups);
   a.uq = a.units / a.G;
   a.ur = a.units % a.G;
   a.part = (float*)workspace;
-  a.up = swiglu ? (bf16*)((char*)workspace + (long long)a.G * 2 * LIN_TILE * sizeof(float)) : nullptr;
-  decode_linear_kernel<<<dim3((unsigned)a.G), 256, 0, st>>>(a);
+  a.up = swiglu ? (bf16*)((char*)workspace + (long long)a.G * 2 * a.pt * sizeof(float)) : nullptr;
+  if (a.tr == 64) decode_linear_kernel<2><<<dim3((unsigned)a.G), 256, 0, st>>>(a);
+  else decode_linear_kernel<1><<<dim3((unsigned)a.G), 256, 0, st>>>(a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(DLLM_ELAUNCH, "decode linear launch: %s", hipGetErrorString(e));
   return DLLM_OK;
@@ -613,7 +647,7 @@ extern "C" int dllm_decode_linear_multi_fwd(const void* x, int M, int K, int cou
   if (rc != DLLM_OK) return rc;
   hipError_t e = hipSuccess;
   if (swiglu) {
-    decode_linear_swiglu_kernel<<<dim3((unsigned)(a.seg[1].tile0 * ((M + 31) / 32)), LIN_FIX_CHUNKS), 256, 0, st>>>(a);
+    decode_linear_swiglu_kernel<<<dim3((unsigned)(a.seg[1].tile0 * ((M + a.tr - 1) / a.tr)), LIN_FIX_CHUNKS * (a.tr / 32)), 256, 0, st>>>(a);
   } else {
     // the tiles a range boundary falls inside, in batches of LIN_FIXMAX
     LinFix f;
@@ -623,7 +657,7 @@ extern "C" int dllm_decode_linear_multi_fwd(const void* x, int M, int K, int cou
       const bool split = b < a.G && ub % a.ns != 0;
       if (split && (f.n == 0 || f.tile[f.n - 1] != ub / a.ns)) f.tile[f.n++] = ub / a.ns;
       if (f.n == LIN_FIXMAX || (b == a.G && f.n > 0)) {
-        decode_linear_fixup_kernel<<<dim3((unsigned)f.n, LIN_FIX_CHUNKS), 256, 0, st>>>(a, f);
+        decode_linear_fixup_kernel<<<dim3((unsigned)f.n, LIN_FIX_CHUNKS * (a.tr / 32)), 256, 0, st>>>(a, f);
         e = hipGetLastError();
         if (e != hipSuccess) break;
         f.n = 0;
@@ -657,7 +691,7 @@ extern "C" int dllm_decode_linear_rmsnorm_fwd(const void* x, const void* weight,
   if (nvw > 8) return fail(DLLM_EUNSUPPORTED, "decode linear rmsnorm: N=%d needs %d vectors per lane (at most 8)", N, nvw);
   // the projection's whole tiles, rounded, go to the workspace after the pieces (the size of
   // dllm_decode_linear_workspace_bytes(M, N, workgroups, 1))
-  void* proj = (char*)workspace + (long long)workgroups * 2 * LIN_TILE * sizeof(float);
+  void* proj = (char*)workspace + (long long)workgroups * 2 * LIN_TILE * (M > 32 ? 2 : 1) * sizeof(float);
   const void* w[1] = {weight};
   void* o[1] = {proj};
   const int n[1] = {N};
@@ -756,14 +790,15 @@ extern "C" int dllm_decode_linear_fwd(const void* x, const void* weight, void* y
 // ---- allocation-free variant: the split-tile pieces live in a fixed per-device array ----------
 //
 // For callers that cannot allocate device memory (code under HIP graph capture, serving loops
-// that forbid it). The pieces a launch needs are G x 2 x 16 KB (two per workgroup), so the array
-// holds 8 MiB = 256 workgroups (one per CU, what dllm_decode_linear_workgroups returns for every
-// projection that splits tiles). Every piece the fixup reads is written by the main kernel of the
+// that forbid it). The pieces a launch needs are G x 2 x 16 KB (two per workgroup), so 8 MiB
+// serve 256 workgroups (one per CU, what dllm_decode_linear_workgroups returns for every projection
+// that splits tiles). More than 32 token rows take tiles, and so pieces, of twice the size (lin_rows,
+// at most 256 workgroups): the array holds twice the 8 MiB that the limit counts. Every piece the fixup reads is written by the main kernel of the
 // same call before it on the same stream, so nothing needs clearing; calls that overlap on one
 // GPU (two streams at once) share the array and race.
 namespace dllm {
 constexpr long long LIN_SCRATCH_BYTES = 8LL << 20;
-static __device__ __align__(256) unsigned char scratch[LIN_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[2 * LIN_SCRATCH_BYTES];
 constexpr int LIN_MAX_DEVICES = 64;
 static void* g_scratch_addr[LIN_MAX_DEVICES];  // device address of `scratch` per device, looked up once
 static std::mutex g_scratch_mu;
@@ -803,7 +838,7 @@ extern "C" int dllm_decode_linear_fwd_noalloc(const void* x, const void* weight,
     return fail(DLLM_EINVAL, "decode linear (no-alloc): bad sizes M=%d N=%d K=%d workgroups=%d", M, N, K, workgroups);
   if (K % 64) return fail(DLLM_EUNSUPPORTED, "decode linear (no-alloc): K=%d is not a multiple of 64", K);
   // the pieces this launch writes: none when every workgroup's unit range is whole tiles
-  const long long units = lin_units(M, (N + 127) / 128, K);
+  const long long units = lin_units(M, (N + 127) / 128, K, 32);
   if (units > 0x7fffffffLL) return fail(DLLM_EUNSUPPORTED, "decode linear (no-alloc): %lld work units is too many", units);
   const long long G = workgroups < units ? workgroups : units;
   const long long ns = K / 64;

@@ -277,7 +277,7 @@ int dllm_block_causal_attention_gated_fwd(const void* q, const int64_t* q_stride
  * denoising step of the reference decoder runs inside block_diffusion_forward
  * (src/dllm_qwen38/decode.py:63-66; [hf]:168-184,656-717) when they see one block of tokens.
  * The launch has `workgroups` workgroups (at most 32768), each streaming an equal share of the
- * (128-feature x 32-row tile, 64-k step) units; dllm_decode_linear_workgroups(M, N, K) gives one per
+ * (128-feature x 32-row tile, 64-k step) units (64-row tiles for more than 32 token rows); dllm_decode_linear_workgroups(M, N, K) gives one per
  * CU, or one per tile when there are at least two tiles per CU (0 if the shape is not taken). Tiles
  * split between workgroups leave fp32 pieces in `workspace` (dllm_decode_linear_workspace_bytes
  * bytes, 16-byte aligned), which a second launch sums in workgroup order: deterministic for a given
@@ -292,8 +292,8 @@ int dllm_decode_linear_fwd(const void* x, const void* weight, void* y, void* wor
  * dllm_decode_linear_fwd without a workspace argument: no counterpart in the reference. For callers
  * that cannot allocate device memory (code under HIP graph capture, serving loops that forbid
  * allocation). The split-tile pieces go to a fixed per-device array inside the library of
- * dllm_decode_linear_noalloc_max_bytes() bytes (8 MiB: 256 workgroups that split tiles, one per
- * CU); a launch needing more returns -2 with a message, and one that splits no tile has no limit.
+ * dllm_decode_linear_noalloc_max_bytes() bytes per 32 token rows (8 MiB: 256 workgroups that split
+ * tiles, one per CU); a launch needing more returns -2 with a message, and one that splits no tile has no limit.
  * Nothing is allocated. The current device must own `stream`. Calls that overlap on one GPU (two
  * streams at once) share the array and race.
  */

@@ -475,3 +475,36 @@ def test_27b_class_cached_step_matches_the_forward_bf16(stack27, dev):
     print(f"27b-class bf16 step vs forward: max|d|={err.max().item():.3e} max|ref|={ref.abs().max().item():.3e}")
     assert (err <= bound).all()
     print(f"cache bytes {cache.nbytes()}")
+
+
+@pytest.mark.parametrize("M,K,N,G", [
+    (33, 320, 300, 1),      # one row past the first 32; every unit in one workgroup
+    (64, 1024, 900, 7),     # whole 64-row tiles, split between workgroups
+    (64, 640, 128 * 260, 256),  # one workgroup per CU, tiles split
+    (50, 640, 128 * 20, 300),   # more than 256 workgroups splitting tiles: 32-row tiles
+    (64, 640, 128 * 20, 20),    # one whole tile per workgroup
+])
+def test_decode_linear_past_32_rows(dev, M, K, N, G):
+    """33 to 64 token rows (64-row tiles, and 32-row tiles past 256 splitting workgroups): the bound of
+    the single-launch test, the first 32 rows' outputs independent of the rows after them within
+    it, and the allocation-free entry point bit-equal."""
+    from dllm_qwen38_amd import _lib
+
+    g = torch.Generator().manual_seed(M + N + G)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16)
+    xd, wd = x.to(dev), w.to(dev)
+    L = _lib.lib()
+    y, y2 = (torch.empty(M, N, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    work = decode._workspace(L, M, 0, G, False, dev)
+    sh = _lib.stream_handle(dev)
+    _lib.check(L.dllm_decode_linear_fwd(xd.data_ptr(), wd.data_ptr(), y.data_ptr(), work.data_ptr(), M, N, K, G,
+                                        _lib.DT_BF16, sh), "decode linear")
+    rc = L.dllm_decode_linear_fwd_noalloc(xd.data_ptr(), wd.data_ptr(), y2.data_ptr(), M, N, K, G, _lib.DT_BF16, sh)
+    torch.cuda.synchronize()
+    ref = x.float() @ w.float().T
+    bound = 2 ** -8 * ref.abs() + 2 ** -16 * (x.float().abs() @ w.float().abs().T)
+    assert ((y.float().cpu() - ref).abs() <= bound).all()
+    assert rc == (-2 if G > 256 else 0)
+    if rc == 0:
+        assert torch.equal(y, y2)
