@@ -543,11 +543,12 @@ struct SpSmem {
 };
 enum { SP_SKIP = 1, SP_RESCALE = 2 };
 
-// TPW: query tiles per workgroup. 4: four consecutive tiles of one query head. 2: two tiles of each
-// of two query heads that share a K/V head (even GQA ratios): the workgroup walks the union of the
+// TPW: query tiles per workgroup. 4: four consecutive tiles of one query head. 2 or 1: two tiles (one
+// tile) of each of two (four) query heads that share a K/V head: the workgroup walks the union of the
 // key tiles its query tiles see, so fewer consecutive tiles waste fewer phases on tiles only some
-// of them see. Every visible tile is walked in the same order either way, so the outputs are the
-// same bits.
+// of them see, and a staged K/V tile serves every one of those heads. Every visible tile is walked in
+// the same order either way, so the outputs are the same bits. With a head count that 4 / TPW does
+// not divide, a K/V head's last workgroup has idle pairs. launch_attn_sp states the choice.
 template <int D, bool BC, int TPW = 4>
 __global__ __launch_bounds__(512) void bd_attn_sp_kernel(AttnArgs a) {
   using SM = SpSmem<D>;
@@ -572,11 +573,11 @@ __global__ __launch_bounds__(512) void bd_attn_sp_kernel(AttnArgs a) {
   const int Lk = BC ? a.N : L;
   const int qa = BC ? a.q0 : 0;
   const int ntq = (Lq + 31) >> 5;
-  static_assert(TPW == 4 || TPW == 2, "query tiles per workgroup");
+  static_assert(TPW == 4 || TPW == 2 || TPW == 1, "query tiles per workgroup");
   constexpr int HPW = 4 / TPW;  // query heads per workgroup
   const int ng = (ntq + TPW - 1) / TPW;
   const int rep = a.Hq / a.Hkv;
-  const int nhu = rep / HPW;    // head units per K/V head
+  const int nhu = (rep + HPW - 1) / HPW;  // head units per K/V head
 
   // work unit: longest first (tile group descending), then half, batch, KV head, query heads in group
   constexpr int NH = BC ? 1 : 2;
@@ -590,11 +591,12 @@ __global__ __launch_bounds__(512) void bd_attn_sp_kernel(AttnArgs a) {
   rem /= nhu;
   const int hkv = rem % a.Hkv;
   const int b = rem / a.Hkv;
-  const int hq = hkv * rep + hr * HPW + pair / TPW;  // this wave pair's query head
+  const int hw = hr * HPW + pair / TPW;  // this wave pair's query head in the group (past the last: idle)
+  const int hq = hkv * rep + min(hw, rep - 1);
 
   const int g0 = g * (32 * TPW), g1 = min(Lq, g0 + 32 * TPW);
   const int r0 = g0 + (pair % TPW) * 32, r1 = min(Lq, r0 + 32);
-  const bool wave_live = r0 < Lq;
+  const bool wave_live = r0 < Lq && hw < rep;
   const int qb0 = (qa + r0) / C, qb1 = (qa + max(r0, r1 - 1)) / C;
   const int gqb0 = (qa + g0) / C, gqb1 = (qa + g1 - 1) / C;
   int lo0, hi0, lo1, hi1;
@@ -784,6 +786,7 @@ __global__ __launch_bounds__(512) void bd_attn_sp_kernel(AttnArgs a) {
       s_phase(n, sa, sb);
       if (n + 1 < nend) s_phase(n + 1, sb, sa);
     }
+    __syncthreads();  // the O waves' barrier before they stage their outputs
     return;
   }
 
@@ -859,100 +862,138 @@ __global__ __launch_bounds__(512) void bd_attn_sp_kernel(AttnArgs a) {
     mfin = *(const float*)(sl + SM::MFIN + 4 * lane);
     lfin = *(const float*)(sl + SM::LFIN + 4 * lane);
   }
+  // Outputs. A lane holds one query's column: storing from the accumulators would write 32 rows in
+  // pieces of 16 (bf16) or 32 bytes per instruction, and read the gate the same way. The rings are
+  // spent, so each O wave turns its 32 rows around in LDS and stores (and reads the gate in) whole
+  // rows, 16 bytes per lane. Pieces against rows:
+  // gated complementary mask at B=2 L=4096, 24 / 4 heads of 256, 1037 -> 1002 us; a 1952-token prompt
+  // 75.0 -> 73.0 us; the decoding step above 25.6 -> 24.1 us.
+  __syncthreads();  // every wave is done with the rings and the slots
+  if (!wave_live) return;
   if constexpr (BC) {
     if (a.ksplit > 1) {  // partial result of this key share, unnormalised (an empty share: zeros)
-      if (wave_live && qi < Lq) {
-        const long long prow = (((long long)blockIdx.y * a.B + b) * Lq + qi) * a.Hq + hq;
-        float* op = a.opart + prow * D;
+      constexpr int SROW = D + 4, LPR = D / 4, RPI4 = 64 / LPR;  // staging row, lanes per row, rows per store
+      static_assert(4 * 32 * SROW * 4 <= SM::TOTAL, "staged rows fit");
+      float* const st = (float*)smem + pair * 32 * SROW;
 #pragma unroll
-        for (int t = 0; t < DT; ++t)
+      for (int t = 0; t < DT; ++t)
 #pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            f32x4 o4;
+        for (int m = 0; m < 4; ++m) {
+          f32x4 o4;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o4[i] = O[t][4 * m + i];
-            *(f32x4*)(op + 32 * t + 8 * m + 4 * h) = o4;
-          }
-        if (h == 0) {
-          a.mlpart[2 * prow] = mfin;
-          a.mlpart[2 * prow + 1] = lfin;
+          for (int i = 0; i < 4; ++i) o4[i] = O[t][4 * m + i];
+          *(f32x4*)(st + l32 * SROW + 32 * t + 8 * m + 4 * h) = o4;
         }
+      const long long prow0 = (((long long)blockIdx.y * a.B + b) * Lq + r0) * a.Hq + hq;  // row r0's; rows Hq apart
+      if (h == 0 && qi < Lq) {
+        const long long prow = prow0 + (long long)l32 * a.Hq;
+        a.mlpart[2 * prow] = mfin;
+        a.mlpart[2 * prow + 1] = lfin;
+      }
+      wave_lds_sync();
+      const int rr = lane / LPR, c = (lane % LPR) * 4;
+#pragma unroll
+      for (int i = 0; i < 32 / RPI4; ++i) {
+        const int row = i * RPI4 + rr;
+        if (r0 + row < Lq)
+          *(f32x4*)(a.opart + (prow0 + (long long)row * a.Hq) * D + c) = *(const f32x4*)(st + row * SROW + c);
       }
       return;
     }
   }
-  if (wave_live && qi < Lq) {
-    const float inv = 1.f / lfin;
-    const long long orow = BC ? (long long)b * Lq + qi : (long long)b * 2 * L + qh * L + qi;
-    bf16* op = (bf16*)a.out + (orow * a.Hq + hq) * a.d;
-    // the output gate (gated attention, [hf]:698): bf16(bf16(o) * bf16(sigmoid(gate))), the
-    // rounding of the separate elementwise product
-    if (a.gate) {
-      // every gate value of the row first (in flight together), then the products;
-      // sigmoid(x) = 1 / (1 + 2^(-x log2 e)) from the hardware exp2 and reciprocal, rounded to bf16
-      const bf16* gp = (const bf16*)a.gate + b * a.g_sb + (long long)(BC ? qi : qh * L + qi) * a.g_st +
-                       (long long)hq * a.g_sh;
-      bf16x4 g4[DT][4];
+  constexpr int SROW = D + 8, RPI8 = 64 / CH, NI = 32 / RPI8;  // staging row, rows per store, stores
+  static_assert(4 * 32 * SROW * 2 <= SM::TOTAL, "staged rows fit");
+  const int rr = lane / CH, c = (lane % CH) * 8;
+  // the output gate (gated attention, [hf]:698): bf16(bf16(o) * bf16(sigmoid(gate))), the rounding of
+  // the separate elementwise product; every gate value first (in flight while the rows are staged)
+  typedef bf16x8 __attribute__((aligned(8))) bf16x8_u;  // gate and output rows: 8-byte aligned
+  bf16x8 g8[NI];
+  if (a.gate) {
+    const bf16* const gp = (const bf16*)a.gate + b * a.g_sb + (long long)((BC ? 0 : qh * L) + r0) * a.g_st +
+                           (long long)hq * a.g_sh + c;
 #pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int m = 0; m < 4; ++m) g4[t][m] = *(const bf16x4*)(gp + 32 * t + 8 * m + 4 * h);
-#pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          bf16x4 o4;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float o = (float)(bf16)(O[t][4 * m + i] * inv);
-            const float sg = (float)(bf16)__builtin_amdgcn_rcpf(
-                1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * (float)g4[t][m][i]));
-            o4[i] = (bf16)(o * sg);
-          }
-          *(bf16x4*)(op + 32 * t + 8 * m + 4 * h) = o4;
-        }
-    } else {
-#pragma unroll
-      for (int t = 0; t < DT; ++t)
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          bf16x4 o4;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) o4[i] = (bf16)(O[t][4 * m + i] * inv);
-          *(bf16x4*)(op + 32 * t + 8 * m + 4 * h) = o4;
-        }
+    for (int i = 0; i < NI; ++i) {
+      const int row = min(i * RPI8 + rr, Lq - 1 - r0);
+      g8[i] = *(const bf16x8_u*)(gp + (long long)row * a.g_st);
     }
+  }
+  bf16* const st = (bf16*)smem + pair * 32 * SROW;
+  const float inv = 1.f / lfin;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      bf16x4 o4;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o4[i] = (bf16)(O[t][4 * m + i] * inv);
+      *(bf16x4*)(st + l32 * SROW + 32 * t + 8 * m + 4 * h) = o4;
+    }
+  wave_lds_sync();
+  const long long orow = BC ? (long long)b * Lq + r0 : (long long)b * 2 * L + qh * L + r0;
+  bf16* const op = (bf16*)a.out + (orow * a.Hq + hq) * D + c;
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int row = i * RPI8 + rr;
+    bf16x8 o8 = *(const bf16x8*)(st + row * SROW + c);
+    if (a.gate) {
+      // sigmoid(x) = 1 / (1 + 2^(-x log2 e)) from the hardware exp2 and reciprocal, rounded to bf16
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float sg = (float)(bf16)__builtin_amdgcn_rcpf(
+            1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * (float)g8[i][e]));
+        o8[e] = (bf16)((float)o8[e] * sg);
+      }
+    }
+    if (r0 + row < Lq) *(bf16x8_u*)(op + (long long)row * a.Hq * D) = o8;
   }
 }
 
 // Merge of the key shares of a split block-causal launch: per (b, query, head) row, with
 // M = max_s m_s and w_s = 2^(m_s - M), out = (sum_s w_s O_s) / (sum_s w_s l_s), times sigmoid(gate)
 // with the main kernel's rounding when a gate is given (row (b, i, h) of [B, M, Hq, d] at
-// b g_sb + i g_st + h g_sh). One thread per four consecutive d.
+// b g_sb + i g_st + h g_sh). One workgroup per row: lane s of every wave holds share s's maximum and
+// sum (at most 64 shares), the 256 threads take D / 4 float4 columns of 1024 / D shares at a time,
+// and the share groups' sums meet in LDS in group order. Bound by latency: one thread per column
+// walking every share in turn, three dependent loads each, took 10.7 us at 17 shares of 768 rows.
+template <int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restrict__ opart,
                                                            const float* __restrict__ mlpart, bf16* __restrict__ out,
-                                                           long long rows, int d, int ks, const bf16* __restrict__ gate,
+                                                           int rows, int ks, const bf16* __restrict__ gate,
                                                            long long g_sb, int g_st, int g_sh, int M, int Hq) {
-  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
-  const int q4 = d / 4;
-  if (t >= rows * q4) return;
-  const long long row = t / q4;
-  const int c = (int)(t % q4) * 4;
-  float mx = -1e30f;
-  for (int s = 0; s < ks; ++s) mx = fmaxf(mx, mlpart[2 * (s * rows + row)]);
-  float l = 0.f;
-  f32x4 o = {0.f, 0.f, 0.f, 0.f};
-  for (int s = 0; s < ks; ++s) {
-    const float w = __builtin_amdgcn_exp2f(mlpart[2 * (s * rows + row)] - mx);
-    l += w * mlpart[2 * (s * rows + row) + 1];
-    const f32x4 p = *(const f32x4*)(opart + (s * rows + row) * d + c);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] += w * p[i];
+  constexpr int Q4 = D / 4, NG = 256 / Q4;  // float4 columns of a row, shares taken at a time
+  __shared__ f32x4 sums[256];
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int grp = tid / Q4, c = (tid % Q4) * 4;
+  float m = -1e30f, l = 0.f;
+  if (lane < ks) {
+    const float* const ml = mlpart + 2 * ((long long)lane * rows + row);
+    m = ml[0];
+    l = ml[1];
   }
-  const float inv = 1.f / l;
+  float mx = m;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  const float w = __builtin_amdgcn_exp2f(m - mx);
+  const float lsum = wave_sum(w * l);
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < ks; s0 += NG) {
+    const int s = s0 + grp;
+    const float ws = __shfl(w, s & 63);  // every lane takes part
+    if (s < ks) {
+      const f32x4 p = *(const f32x4*)(opart + ((long long)s * rows + row) * D + c);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o[i] += ws * p[i];
+    }
+  }
+  sums[tid] = o;
+  __syncthreads();
+  if (grp != 0) return;
+#pragma unroll
+  for (int g = 1; g < NG; ++g) o += sums[g * Q4 + tid];
+  const float inv = 1.f / lsum;
   bf16x4 r;
   if (gate) {
-    const long long bi = row / Hq;  // b M + i
+    const int bi = row / Hq;  // b M + i
     const bf16x4 g4 = *(const bf16x4*)(gate + (bi / M) * g_sb + (long long)(bi % M) * g_st +
                                        (long long)(row % Hq) * g_sh + c);
 #pragma unroll
@@ -965,29 +1006,37 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
 #pragma unroll
     for (int i = 0; i < 4; ++i) r[i] = (bf16)(o[i] * inv);
   }
-  *(bf16x4*)(out + row * d + c) = r;
+  *(bf16x4*)(out + (long long)row * D + c) = r;
 }
 
 template <int D, bool BC>
 static int launch_attn_sp(const AttnArgs& a, hipStream_t st) {
   const int ntq = ((BC ? a.M : a.L) + 31) / 32;
-  // two query heads per workgroup where the GQA ratio is even (complementary-mask mode; measured
-  // 911.6 vs 947.2 us at B=2 L=4096 Hq=24 Hkv=4 d=256, bit-identical)
-  const bool two = !BC && (a.Hq / a.Hkv) % 2 == 0;
-  const int tpw = two ? 2 : 4;
-  const int ng = (ntq + tpw - 1) / tpw;
-  const long long nblk = (long long)ng * (BC ? 1 : 2) * a.B * a.Hq / (4 / tpw);
-  if (nblk > 0x7fffffff) return fail(DLLM_EUNSUPPORTED, "attention: grid too large");
+  const int rep = a.Hq / a.Hkv;
   const int ks = BC && a.ksplit > 1 ? a.ksplit : 1;
-  if (two) bd_attn_sp_kernel<D, BC, 2><<<dim3((unsigned)nblk, ks), dim3(512), 0, st>>>(a);
-  else bd_attn_sp_kernel<D, BC, 4><<<dim3((unsigned)nblk, ks), dim3(512), 0, st>>>(a);
+  // One query tile (a decoding step): four query heads per workgroup where the key tiles are split or
+  // the heads alone would fill the chip (a K/V tile is then staged once for the four; B=1 M=32
+  // N=4128, 24 / 4 heads of 256, both launches: 41.2 us with a workgroup per head, 24.1 with four
+  // heads); a short unsplit step is latency, which four heads on one CU lengthen (N=64: 12.0 vs
+  // 10.2 us). More tiles: two heads where the GQA ratio is even (complementary mask 911.6 vs
+  // 947.2 us at B=2 L=4096 of the same heads, a prompt of 1952 tokens 75 vs 82 us).
+  const bool share = ks > 1 || (BC ? 1LL : 2LL) * a.B * a.Hq > 256;
+  const int tpw = ntq == 1 ? (rep > 1 && share ? 1 : 4) : rep % 2 == 0 ? 2 : 4;
+  const int nhu = (rep + 4 / tpw - 1) / (4 / tpw);
+  const int ng = (ntq + tpw - 1) / tpw;
+  const long long nblk = (long long)ng * (BC ? 1 : 2) * a.B * a.Hkv * nhu;
+  if (nblk > 0x7fffffff) return fail(DLLM_EUNSUPPORTED, "attention: grid too large");
+  const long long rows = (long long)a.B * a.M * a.Hq;  // block-causal mode
+  if (ks > 1 && rows > 0x7fffffff) return fail(DLLM_EUNSUPPORTED, "attention: grid too large");
+  const dim3 grid((unsigned)nblk, ks);
+  if (tpw == 1) bd_attn_sp_kernel<D, BC, 1><<<grid, dim3(512), 0, st>>>(a);
+  else if (tpw == 2) bd_attn_sp_kernel<D, BC, 2><<<grid, dim3(512), 0, st>>>(a);
+  else bd_attn_sp_kernel<D, BC, 4><<<grid, dim3(512), 0, st>>>(a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(DLLM_ELAUNCH, "attention launch: %s", hipGetErrorString(e));
   if (ks > 1) {
-    const long long rows = (long long)a.B * a.M * a.Hq;
-    const long long n = rows * (D / 4);
-    attn_combine_kernel<<<dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st>>>(
-        a.opart, a.mlpart, (bf16*)a.out, rows, D, ks, (const bf16*)a.gate, a.g_sb, a.g_st, a.g_sh, a.M, a.Hq);
+    attn_combine_kernel<D><<<dim3((unsigned)rows), dim3(256), 0, st>>>(
+        a.opart, a.mlpart, (bf16*)a.out, (int)rows, ks, (const bf16*)a.gate, a.g_sb, a.g_st, a.g_sh, a.M, a.Hq);
     e = hipGetLastError();
     if (e != hipSuccess) return fail(DLLM_ELAUNCH, "attention combine launch: %s", hipGetErrorString(e));
   }

@@ -124,12 +124,21 @@ def bd_attention_gated(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, gate: 
     return out
 
 
-def _key_splits(q: torch.Tensor, M: int, N: int, d: int) -> int:
-    """Key splits for a decoding step (bf16, the direct-load kernel's head sizes, few query rows):
-    about eight 32-key tiles per workgroup; 1 otherwise."""
-    if q.dtype != torch.bfloat16 or d not in (64, 128, 256) or M > 64 or N < 512:
+def _key_splits(q: torch.Tensor, M: int, N: int, Hkv: int, d: int) -> int:
+    """Key splits for a decoding step (bf16, the direct-load kernel's head sizes, few query rows); 1
+    otherwise. A K/V head's query heads run four (M <= 32) or two to a workgroup, so one share has
+    B * Hkv * ceil(rep / 4) workgroups or so: as many shares as fit one workgroup per CU (past it a
+    second round costs more than shorter shares save: at B = 4, N = 4128, 24 / 4 heads of 256, 8
+    shares 39.3 us, 16 53.0), of about four 32-key tiles each (fewer tiles save less than their
+    part of the merge costs: at B = 1, N = 2080, 12 to 20 shares 23.8-24.1 us, 8 25.5, 64 37.3). Up
+    to 160 keys one share is as fast (N = 160: 13.1 us, two shares 13.9)."""
+    tiles = -(-N // 32)
+    if q.dtype != torch.bfloat16 or d not in (64, 128, 256) or M > 64 or tiles <= 5:
         return 1
-    return max(1, min(32, -(-N // 256)))
+    B, rep = q.shape[0], q.shape[2] // Hkv
+    hpw = 1 if rep == 1 else 4 if M <= 32 else 2 if rep % 2 == 0 else 1
+    units = B * Hkv * -(-rep // hpw)
+    return max(1, min(64, 256 // units, -(-tiles // 4)))
 
 
 def block_causal_gate_fused(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
@@ -175,7 +184,7 @@ def block_causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     if B == 0 or M == 0:  # no queries: an empty output, no launch
         return out
     sc = d ** -0.5 if scale is None else float(scale)
-    ks = _key_splits(q, M, N, d) if key_splits is None else int(key_splits)
+    ks = _key_splits(q, M, N, Hkv, d) if key_splits is None else int(key_splits)
     work = torch.empty(ks * B * M * Hq * (d + 2), dtype=torch.float32, device=dev) if ks > 1 else None
     if gate is not None:
         if tuple(gate.shape) != (B, M, Hq, d) or gate.dtype != q.dtype or gate.stride(-1) != 1:

@@ -508,3 +508,24 @@ def test_decode_linear_past_32_rows(dev, M, K, N, G):
     assert rc == (-2 if G > 256 else 0)
     if rc == 0:
         assert torch.equal(y, y2)
+
+
+@pytest.mark.parametrize("B,M,N,Hq,Hkv,d,block", [
+    (1, 32, 288, 12, 2, 256, 32),   # six heads of a K/V head in two workgroups, one of them half idle; 2 shares
+    (2, 8, 1000, 5, 1, 64, 8),      # five heads, ragged query tile and key tiles
+    (1, 17, 700, 8, 1, 128, 17),    # eight heads: two full workgroups
+    (1, 64, 1024, 6, 2, 256, 32),   # two query tiles: two heads per workgroup, the third with an idle pair
+    (3, 1, 2080, 4, 4, 128, 1),     # one head per K/V head, one query row
+    (1, 200, 200, 12, 2, 256, 8),   # a prompt, two heads per workgroup, ragged last tiles
+])
+def test_block_causal_heads_sharing_a_workgroup(dev, B, M, N, Hq, Hkv, d, block):
+    """Query heads that share staged K/V tiles, over head counts that do not fill a workgroup, with
+    the default key shares, 64 (the most; many of them empty) and one: within the bf16 bar of the
+    oracle."""
+    q, k, v = _att_inputs(B, M, N, Hq, Hkv, d, torch.bfloat16, seed=M + N + Hq)
+    ref = attn_ref.block_causal_attention(q, k, v, block=block, q_offset=N - M)
+    qd, kd, vd = q.to(dev), k.to(dev), v.to(dev)
+    for ks in (None, 64, 1):
+        got = attention.block_causal_attention(qd, kd, vd, block=block, q_offset=N - M, key_splits=ks)
+        torch.cuda.synchronize()
+        _check_att(got, ref, torch.bfloat16, v.float().abs().max().item(), f"M{M} N{N} {Hq}/{Hkv} shares {ks}")
