@@ -1019,9 +1019,12 @@ static int launch_attn_sp(const AttnArgs& a, hipStream_t st) {
   // N=4128, 24 / 4 heads of 256, both launches: 41.2 us with a workgroup per head, 24.1 with four
   // heads); a short unsplit step is latency, which four heads on one CU lengthen (N=64: 12.0 vs
   // 10.2 us). More tiles: two heads where the GQA ratio is even (complementary mask 911.6 vs
-  // 947.2 us at B=2 L=4096 of the same heads, a prompt of 1952 tokens 75 vs 82 us).
+  // 947.2 us at B=2 L=4096 of the same heads, a prompt of 1952 tokens 75 vs 82 us), but for a prompt
+  // whose workgroups of one head fit the chip at once, where the heads apart are as long and load
+  // K/V beside each other (576 tokens 27.5 vs 29.2 us).
   const bool share = ks > 1 || (BC ? 1LL : 2LL) * a.B * a.Hq > 256;
-  const int tpw = ntq == 1 ? (rep > 1 && share ? 1 : 4) : rep % 2 == 0 ? 2 : 4;
+  const bool fits = BC && ks == 1 && (long long)((ntq + 3) / 4) * a.B * a.Hq <= 256;
+  const int tpw = ntq == 1 ? (rep > 1 && share ? 1 : 4) : rep % 2 == 0 && !fits ? 2 : 4;
   const int nhu = (rep + 4 / tpw - 1) / (4 / tpw);
   const int ng = (ntq + tpw - 1) / tpw;
   const long long nblk = (long long)ng * (BC ? 1 : 2) * a.B * a.Hkv * nhu;

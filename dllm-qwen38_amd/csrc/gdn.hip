@@ -29,76 +29,9 @@
 
 #include <atomic>
 
-#include "common.h"
+#include "gdn_common.h"
 
 namespace dllm {
-
-struct GdnStream {
-  const void* q;
-  const void* k;
-  const void* v;
-  const float* beta;
-  const float* g;
-  void* out;  // [B, T, Hv, Dv] contiguous
-};
-
-struct GdnArgs {
-  GdnStream s[2];
-  const float* init;  // [B, Hv, Dk, Dv] fp32 or null
-  float* states;      // [B, T/chunk, Hv, Dk, Dv] fp32 or null
-  long long q_sb, k_sb, v_sb, b_sb, g_sb;  // batch strides (elements)
-  int q_st, q_sh, k_st, k_sh, v_st, v_sh, b_st, b_sh, g_st, g_sh;  // token / head strides
-  int B, T, Hk, Hv, Dk, Dv;
-  int sub;         // real rows per 32-row tile
-  int snap_every;  // tiles per chunk
-  float scale;     // applied to q after l2norm
-  int l2norm;
-  int vec_qk;  // q/k rows: 16-byte vector loads (aligned, Dk equal to the kernel width)
-  int vec_v;   // v rows: 16-byte vector loads (aligned, Dv a multiple of the column window)
-  int spin_limit;  // bounded waits give up (and report through dllm_status) after this many sleeps
-  int wait_bias;   // 0; tests set a count the LDS wait never reaches, to exercise the give-up path
-  // pipelined fork over a range of blocks: rows and snapshots per sequence of the full out and
-  // states tensors (T and T / sub for a whole sequence), and the clean state the range starts
-  // from (the snapshot of the block before it, in the states layout; null: zeros)
-  int t_rows, snap_rows;
-  const float* fork_init;
-  // pipelined fork with the v channels' causal conv (width 4) + SiLU in the state waves: the v rows
-  // read are the conv's inputs; weights [Hv * Dv, 4] (the v channels' rows; bf16, or fp32 in the
-  // kernel's fp32-weight instantiation) and bias [Hv * Dv] of the same dtype, or null. t_first: the
-  // sequence row of the launch's first row (the history before sequence row 0 is zero).
-  const void* vconv_w;
-  const void* vconv_b;
-  int t_first;
-  // the v channels' conv tails (the clean raw rows before each block, [B * nb, tails_cd, 3] from the
-  // first v channel on), or null
-  void* vtails;
-  int tails_cd;
-};
-
-// Linear workgroup id such that consecutive ids run on the same XCD (dispatch is round-robin over
-// the 8 XCDs): workgroups sharing a key head then share that XCD's L2.
-__device__ __forceinline__ int xcd_linear_id(int bid, int n) {
-  const int q = n >> 3, r = n & 7, x = bid & 7, i = bid >> 3;
-  return (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
-}
-
-// Returns x unchanged but opaque to the optimiser, so that uniform addresses derived from it are
-// computed where they are used instead of being hoisted out of the tile loop (and spilled).
-__device__ __forceinline__ int opaque(int x) {
-  asm volatile("" : "+s"(x));
-  return x;
-}
-// The same for a per-lane value: comparisons against it are evaluated where they are used instead
-// of being hoisted out of the tile loop as lane masks held in (spilled) scalar registers.
-__device__ __forceinline__ int opaque_v(int x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
-
-// DPP move; lanes whose source is outside the row read 0 (bound_ctrl).
-template <int CTRL> __device__ __forceinline__ float dpp_mov(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
-}
 
 // Sum over each aligned group of 8 lanes, returned to all 8 (DPP: no LDS round trip). The three
 // steps are quad_perm [1,0,3,2], quad_perm [2,3,0,1] and row_half_mirror.
@@ -763,58 +696,6 @@ __global__ __launch_bounds__(FORK ? 512 : 256) void gdn_chunk_kernel(GdnArgs a) 
 // same LDS counter, which the state waves raise after reading the staged rows.
 // One barrier per tile; every operand the roles exchange is double-buffered by tile parity. Each
 // SIMD runs one state wave beside one G or P wave.
-// Sum of squares of row l32 of a [32 x 128] bf16 operand held as four rho-ordered fragments (lane
-// (l32, h) holds 64 of the row's values): paired bf16 dot products into four fp32 partial sums,
-// then the other half of the row from lane l32 + 32 (or l32 - 32), so both lanes get the row total.
-__device__ __forceinline__ float row_sumsq(const Frag<true> (&f)[4]) {
-  float s[4];
-#pragma unroll
-  for (int kt = 0; kt < 4; ++kt) {
-    float x = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const bf16x2 lo = {f[kt].lo[2 * i], f[kt].lo[2 * i + 1]};
-      const bf16x2 hi = {f[kt].hi[2 * i], f[kt].hi[2 * i + 1]};
-      x = __builtin_amdgcn_fdot2_f32_bf16(lo, lo, x, false);
-      x = __builtin_amdgcn_fdot2_f32_bf16(hi, hi, x, false);
-    }
-    s[kt] = x;
-  }
-  const float half = (s[0] + s[1]) + (s[2] + s[3]);
-  // the other half from lane l ^ 32 (LDS crossbar permute); the sum is commutative, so the two
-  // lanes of a row hold bit-identical totals
-  const float other = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute((__lane_id() ^ 32) << 2,
-                                                                            __builtin_bit_cast(int, half)));
-  return half + other;
-}
-
-// Pipelined-kernel operand convention. The state S is held with its rows (d) permuted inside each
-// 32-row slice: accumulator row rho(v, h) holds d = 16 h + v. Fed back as a B operand, value v of
-// lane (n, h) then carries d = 16 h + v, so every A operand contracted with it (W, Q) is read as 16
-// CONSECUTIVE d of its row: two 16-byte LDS reads instead of four 8-byte ones. Products whose two
-// operands both come from LDS rows (K K^T, K Q^T) use the same reads for both: the contraction pairs
-// equal d whatever the order.
-__device__ __forceinline__ void lds_frag_c(const bf16* base, int h, Frag<true>& f) {
-  const bf16* p = base + 16 * h;
-  f.lo = *(const bf16x8*)p;
-  f.hi = *(const bf16x8*)(p + 8);
-}
-// Transposed read (as lds_frag_tr) whose result lane r = 8 m + 4 h' + e receives column
-// 16 h' + 4 m + e of the 32-column slice: an A operand whose product rows come out in the permuted
-// d order above. The transpose read hands each group of four result lanes the four consecutive
-// columns one source lane addresses, so only the column-group addresses change.
-__device__ __forceinline__ void lds_frag_tr_d(const bf16* base, int row_stride, int lane, Frag<true>& f) {
-  typedef __attribute__((address_space(3))) bf16x4 lds_bf16x4;
-  const int s = lane & 15, j = s & 3;
-  const bf16* p = base + (4 * (lane >> 5) + (s >> 2)) * row_stride + 16 * (j & 1) + 4 * (2 * ((lane >> 4) & 1) + (j >> 1));
-  bf16x4 r[4];
-#pragma unroll
-  for (int m = 0; m < 4; ++m)
-    r[m] = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)(p + 8 * m * row_stride));
-  f.lo = __builtin_shufflevector(r[0], r[1], 0, 1, 2, 3, 4, 5, 6, 7);
-  f.hi = __builtin_shufflevector(r[2], r[3], 0, 1, 2, 3, 4, 5, 6, 7);
-}
-
 struct PipeSmem {
   static constexpr int DK = 128;
   static constexpr int QROW = DK + 8;          // bf16 row stride of q, k, W and v rows
@@ -863,42 +744,6 @@ enum { VG_BR = 0, VG_C1 = 32 };
 // the pipelined fork gave up (the launch's outputs are then invalid).
 enum { STATUS_LDS_WAIT = 1u };
 static __device__ unsigned dllm_status_word;
-
-// One fp32 element of a state snapshot: a non-temporal store (nothing in the launch reads the
-// snapshot back) at device scope, so that the line is written through to memory instead of held
-// dirty in the XCD's L2 until the launch ends. Issued as its own instruction, which also keeps the
-// compiler from moving the stores among the update's products. Measured at the 27B-class layer:
-// the fork 559.6 vs 594.3 us with the compiler's non-temporal store (571.2 us for the same nt
-// store issued this way, 562.3 us with system scope), bit-identical; 253.1 vs 259.2 us at the
-// 0.8B-class layer.
-// OFF: an immediate byte offset from p.
-template <int OFF> __device__ __forceinline__ void store_snapshot(float* p, float v) {
-  asm volatile("global_store_dword %0, %1, off offset:%2 nt sc1" ::"v"(p), "v"(v), "i"(OFF) : "memory");
-}
-// The 16 values of one 32-row slice of a state wave's accumulator: rows 32 kt + 16 h + v of the
-// snapshot (p0 = row 32 kt + 16 h), 512 bytes apart, as immediate offsets from two base addresses
-// (v < 8 and v >= 8) instead of an address formed per store. With the v conv on the state waves
-// (whose VALU is then the bound) this measured 604 vs 611 us at the 27B-class fork and 260 vs
-// 270 us at the 0.8B-class, bit-identical (before it: 581 vs 561 us, slower).
-__device__ __forceinline__ void store_snapshot_slice(float* p0, const f32x16& s) {
-  float* const p1 = p0 + 8 * 128;
-  store_snapshot<0>(p0, s[0]);
-  store_snapshot<512>(p0, s[1]);
-  store_snapshot<1024>(p0, s[2]);
-  store_snapshot<1536>(p0, s[3]);
-  store_snapshot<2048>(p0, s[4]);
-  store_snapshot<2560>(p0, s[5]);
-  store_snapshot<3072>(p0, s[6]);
-  store_snapshot<3584>(p0, s[7]);
-  store_snapshot<0>(p1, s[8]);
-  store_snapshot<512>(p1, s[9]);
-  store_snapshot<1024>(p1, s[10]);
-  store_snapshot<1536>(p1, s[11]);
-  store_snapshot<2048>(p1, s[12]);
-  store_snapshot<2560>(p1, s[13]);
-  store_snapshot<3072>(p1, s[14]);
-  store_snapshot<3584>(p1, s[15]);
-}
 
 __device__ __forceinline__ void report_status(unsigned bit) {
   __hip_atomic_fetch_or(&dllm_status_word, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1132,101 +977,7 @@ __global__ __launch_bounds__(512) void gdn_fork_pipe_kernel(GdnArgs a) {
               AF[i * FROW + l32] = (lo < 8 * m + 4 * ho + e) ? val : 0.f;
             }
           wave_lds_sync();
-          // level 0: four 8x8 diagonal blocks, one column per lane (lanes 0..31); lanes of odd
-          // blocks also clear the block above (read as zero by level 2)
-          if (h == 0) {
-            const int bb = l32 >> 3, cc = lo & 7, o = 8 * bb;
-            f32x4 ar[8][2];
-#pragma unroll
-            for (int i = 1; i < 8; ++i) {
-              ar[i][0] = *(const f32x4*)(AF + (o + i) * FROW + o);
-              ar[i][1] = *(const f32x4*)(AF + (o + i) * FROW + o + 4);
-            }
-            float x[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) x[i] = (i == cc) ? 1.f : 0.f;
-#pragma unroll
-            for (int i = 1; i < 8; ++i) {
-              float sacc = 0.f;
-#pragma unroll
-              for (int j = 0; j < i; ++j) sacc = __builtin_fmaf(ar[i][j >> 2][j & 3], x[j], sacc);
-              if (i > cc) x[i] = -sacc;
-            }
-#pragma unroll
-            for (int i = 0; i < 8; ++i) TF[(o + i) * FROW + o + cc] = x[i];
-            if (bb & 1) {
-#pragma unroll
-              for (int i = 0; i < 8; ++i) TF[(o - 8 + i) * FROW + o + cc] = 0.f;
-            }
-          }
-          wave_lds_sync();
-          // level 1: T[m+1][m] = -D[m+1] (A[m+1][m] D[m]) for the sub-diagonal 8x8 blocks m = 0 and 2
-          // (inside the 16x16 diagonal blocks; the block m = 1 lies in T[16:32][0:16], which level 2
-          // writes whole without reading it)
-          {
-            const int ii = lane >> 3, jj = lane & 7;
-            f32x4 arow[2][2];
-            float dcol[2][8];
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-              const int m = 2 * q;
-              arow[q][0] = *(const f32x4*)(AF + (8 * (m + 1) + ii) * FROW + 8 * m);
-              arow[q][1] = *(const f32x4*)(AF + (8 * (m + 1) + ii) * FROW + 8 * m + 4);
-#pragma unroll
-              for (int kk = 0; kk < 8; ++kk) dcol[q][kk] = TF[(8 * m + kk) * FROW + 8 * m + jj];
-            }
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-              float sacc = 0.f;
-#pragma unroll
-              for (int kk = 0; kk < 8; ++kk) sacc = __builtin_fmaf(arow[q][kk >> 2][kk & 3], dcol[q][kk], sacc);
-              YF[q * 64 + ii * 8 + jj] = sacc;
-            }
-            wave_lds_sync();
-            f32x4 drow[2][2];
-            float ycol[2][8];
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-              const int m = 2 * q;
-              drow[q][0] = *(const f32x4*)(TF + (8 * (m + 1) + ii) * FROW + 8 * (m + 1));
-              drow[q][1] = *(const f32x4*)(TF + (8 * (m + 1) + ii) * FROW + 8 * (m + 1) + 4);
-#pragma unroll
-              for (int kk = 0; kk < 8; ++kk) ycol[q][kk] = YF[q * 64 + kk * 8 + jj];
-            }
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-              const int m = 2 * q;
-              float sacc = 0.f;
-#pragma unroll
-              for (int kk = 0; kk < 8; ++kk) sacc = __builtin_fmaf(drow[q][kk >> 2][kk & 3], ycol[q][kk], sacc);
-              TF[(8 * (m + 1) + ii) * FROW + 8 * m + jj] = -sacc;
-            }
-          }
-          wave_lds_sync();
-          // level 2: T[16:32][0:16] = -T22 (A21 T11) as fp32 16x16x4 matrix products (lane l supplies
-          // A[l % 16][l / 16] and B[l / 16][l % 16] and holds D[4 (l / 16) + v][l % 16]), the
-          // intermediate through YF; on the VALU this level was 128 FMAs per lane, on a SIMD whose
-          // VALU the state wave beside it needs (27B-class fork 623 vs 649 us; the outputs measured
-          // bit-identical to the FMA form, whose sums ran in the same k order)
-          {
-            const int li = lane & 15, lk = lane >> 4;
-            f32x4 y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
-              y = __builtin_amdgcn_mfma_f32_16x16x4f32(AF[(16 + li) * FROW + 4 * kb + lk], TF[(4 * kb + lk) * FROW + li], y,
-                                                       0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) YF[(4 * lk + v) * 20 + li] = y[v];
-            wave_lds_sync();
-            f32x4 z = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
-              z = __builtin_amdgcn_mfma_f32_16x16x4f32(TF[(16 + li) * FROW + 16 + 4 * kb + lk], YF[(4 * kb + lk) * 20 + li],
-                                                       z, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) TF[(16 + 4 * lk + v) * FROW + li] = -z[v];
-          }
-          wave_lds_sync();
+#include "gdn_inverse.inc"
           // T1 = T diag(beta e^gamma / ||k||) and T2 = T diag(beta) as operand fragments
           // (lane = row l32, columns rho(v, h); lower triangle with the diagonal)
           f32x16 tv1, tv2;
@@ -1766,11 +1517,42 @@ extern "C" int dllm_gdn_state_fork_path(int Dk, int Dv, int block, int dtype) {
   return (dtype == DT_BF16 && Dk == 128 && Dv == 128) ? 2 : 1;
 }
 
+// The prepared-tile path (gdn_scan.hip) takes 128 x 128 bf16 heads, blocks that divide the 32-row tile,
+// few (sequence, head) pairs and at least ten tiles; its workspace in bytes, 0 where it is not taken.
+extern "C" long long dllm_gdn_scan_workspace_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, int dtype,
+                                                   int streams, int states) {
+  if (B <= 0 || T <= 0 || Hk <= 0 || Hv <= 0 || chunk <= 0 || Hv % Hk || T % chunk || 32 % chunk) return 0;
+  if (dtype != DT_BF16 || Dk != 128 || Dv != 128 || (streams != 1 && streams != 2)) return 0;
+  return gdn_scan_workspace(B, T, Hk, Hv, chunk, streams, states != 0, nullptr);
+}
+
+// Whether the prepared-tile path runs: shape (need > 0) and a workspace for it. A workspace that is too
+// small or misaligned is an error (sets *rc).
+static bool scan_taken(long long need, void* workspace, long long workspace_bytes, int* rc) {
+  *rc = DLLM_OK;
+  if (!workspace || need == 0) return false;
+  if (workspace_bytes < need || ((uintptr_t)workspace & 255))
+    *rc = fail(DLLM_EINVAL, "gdn: the workspace must be 256-byte aligned and hold %lld bytes (%lld given)", need,
+               workspace_bytes);
+  return true;
+}
+
 extern "C" int dllm_gdn_chunk_fwd(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
                                   const void* v, const int64_t* v_strides, const float* g, const int64_t* g_strides,
                                   const float* beta, const int64_t* beta_strides, const float* initial_state,
                                   void* out, float* states, int B, int T, int Hk, int Hv, int Dk, int Dv,
                                   int chunk, int dtype, int use_qk_l2norm, float scale, void* stream) {
+  return dllm_gdn_chunk_ws_fwd(q, q_strides, k, k_strides, v, v_strides, g, g_strides, beta, beta_strides,
+                               initial_state, out, states, B, T, Hk, Hv, Dk, Dv, chunk, dtype, use_qk_l2norm, scale,
+                               nullptr, 0, stream);
+}
+
+extern "C" int dllm_gdn_chunk_ws_fwd(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                                     const void* v, const int64_t* v_strides, const float* g, const int64_t* g_strides,
+                                     const float* beta, const int64_t* beta_strides, const float* initial_state,
+                                     void* out, float* states, int B, int T, int Hk, int Hv, int Dk, int Dv,
+                                     int chunk, int dtype, int use_qk_l2norm, float scale, void* workspace,
+                                     long long workspace_bytes, void* stream) {
   if (!q || !k || !v || !g || !beta || !out || !q_strides || !k_strides || !v_strides || !g_strides || !beta_strides)
     return fail(DLLM_EINVAL, "gdn: null pointer");
   if (B <= 0 || T <= 0 || Hk <= 0 || Hv <= 0 || Dk <= 0 || Dv <= 0 || chunk <= 0)
@@ -1814,6 +1596,10 @@ extern "C" int dllm_gdn_chunk_fwd(const void* q, const int64_t* q_strides, const
     a.t_rows = T;
     a.snap_rows = T / a.sub;
     a.fork_init = nullptr;
+    int rc;
+    if (scan_taken(dllm_gdn_scan_workspace_bytes(B, T, Hk, Hv, Dk, Dv, chunk, dtype, 1, states != nullptr), workspace,
+                   workspace_bytes, &rc))
+      return rc == DLLM_OK ? gdn_scan_launch(a, 1, workspace, (hipStream_t)stream) : rc;
     return launch_fork_pipe<1>(a, (hipStream_t)stream);
   }
   return dispatch_gdn(a, dtype, false, (hipStream_t)stream);
@@ -1836,7 +1622,8 @@ struct VConv {
 static int state_fork(const void* qkv0, const void* qkvt, int64_t qkv_stride_b, int64_t qkv_stride_t,
                       const float* beta0, const float* betat, const float* g0, const float* gt, void* out0,
                       void* outt, float* states, int B, int L, int Hk, int Hv, int Dk, int Dv, int block, int dtype,
-                      float scale, int kb0, int kb1, void* stream, const VConv* vc = nullptr) {
+                      float scale, int kb0, int kb1, void* stream, const VConv* vc = nullptr,
+                      void* workspace = nullptr, long long workspace_bytes = 0) {
   if (!qkv0 || !qkvt || !beta0 || !betat || !g0 || !gt || !out0 || !outt) return fail(DLLM_EINVAL, "gdn fork: null pointer");
   if (vc) {
     if (!vc->raw0 || !vc->rawt || !vc->weight) return fail(DLLM_EINVAL, "gdn fork v conv: null pointer");
@@ -1923,7 +1710,13 @@ static int state_fork(const void* qkv0, const void* qkvt, int64_t qkv_stride_b, 
                                  : launch_fork_pipe<2, 1>(a, (hipStream_t)stream);
   }
   // full 128 x 128 heads with 16-byte rows: the pipelined kernel
-  if (dtype == DT_BF16 && Dk == 128 && Dv == 128 && a.vec_qk && a.vec_v) return launch_fork_pipe<2>(a, (hipStream_t)stream);
+  if (dtype == DT_BF16 && Dk == 128 && Dv == 128 && a.vec_qk && a.vec_v) {
+    int rc;
+    if (whole && scan_taken(dllm_gdn_scan_workspace_bytes(B, L, Hk, Hv, Dk, Dv, block, dtype, 2, states != nullptr), workspace,
+                            workspace_bytes, &rc))
+      return rc == DLLM_OK ? gdn_scan_launch(a, 2, workspace, (hipStream_t)stream) : rc;
+    return launch_fork_pipe<2>(a, (hipStream_t)stream);
+  }
   if (!whole) return fail(DLLM_EUNSUPPORTED, "gdn fork: block ranges need the pipelined kernel (bf16, Dk = Dv = 128)");
   return dispatch_gdn(a, dtype, true, (hipStream_t)stream);
 }
@@ -1935,6 +1728,16 @@ extern "C" int dllm_gdn_state_fork_fwd(const void* qkv0, const void* qkvt, int64
   const int nb = block > 0 && L > 0 && L % block == 0 ? L / block : 1;  // sizes are checked by state_fork
   return state_fork(qkv0, qkvt, qkv_stride_b, qkv_stride_t, beta0, betat, g0, gt, out0, outt, states, B, L, Hk, Hv,
                     Dk, Dv, block, dtype, scale, 0, nb, stream);
+}
+
+extern "C" int dllm_gdn_state_fork_ws_fwd(const void* qkv0, const void* qkvt, int64_t qkv_stride_b, int64_t qkv_stride_t,
+                                          const float* beta0, const float* betat, const float* g0, const float* gt,
+                                          void* out0, void* outt, float* states, int B, int L, int Hk, int Hv, int Dk,
+                                          int Dv, int block, int dtype, float scale, void* workspace,
+                                          long long workspace_bytes, void* stream) {
+  const int nb = block > 0 && L > 0 && L % block == 0 ? L / block : 1;  // sizes are checked by state_fork
+  return state_fork(qkv0, qkvt, qkv_stride_b, qkv_stride_t, beta0, betat, g0, gt, out0, outt, states, B, L, Hk, Hv,
+                    Dk, Dv, block, dtype, scale, 0, nb, stream, nullptr, workspace, workspace_bytes);
 }
 
 extern "C" int dllm_gdn_state_fork_range_fwd(const void* qkv0, const void* qkvt, int64_t qkv_stride_b,

@@ -33,6 +33,15 @@ _SIGNATURES = {
         _c_void_p, _c_i64p, _c_void_p, _c_i64p, _c_void_p, _c_i64p, _c_fp, _c_i64p, _c_void_p, _c_i64p,
         _c_fp, _c_void_p, _c_fp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
         _c_float, _c_void_p]),
+    "dllm_gdn_scan_workspace_bytes": (_c_i64, [_c_int] * 10),
+    "dllm_gdn_chunk_ws_fwd": (_c_int, [
+        _c_void_p, _c_i64p, _c_void_p, _c_i64p, _c_void_p, _c_i64p, _c_fp, _c_i64p, _c_void_p, _c_i64p,
+        _c_fp, _c_void_p, _c_fp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+        _c_float, _c_void_p, _c_i64, _c_void_p]),
+    "dllm_gdn_state_fork_ws_fwd": (_c_int, [
+        _c_void_p, _c_void_p, _c_i64, _c_i64, _c_void_p, _c_void_p, _c_fp, _c_fp, _c_void_p, _c_void_p,
+        _c_fp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void_p, _c_i64,
+        _c_void_p]),
     "dllm_gdn_fused_fork_supported": (_c_int, [_c_int, _c_int, _c_int]),
     "dllm_gdn_state_fork_path": (_c_int, [_c_int, _c_int, _c_int, _c_int]),
     "dllm_set_spin_limit": (_c_int, [_c_int]),

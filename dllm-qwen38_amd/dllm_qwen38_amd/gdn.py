@@ -97,13 +97,24 @@ def chunk_gated_delta_rule_with_states(
         _IMPL["last"], _IMPL["reason"] = "hip", "empty input"
         return out, states
     L = _lib.lib()
-    _lib.check(L.dllm_gdn_chunk_fwd(
+    # a decoding step's few tiles never take a workspace: not asked for there
+    ws, nws = (None, 0) if T < 10 * chunk_size else _scan_workspace(L, dev, B, T, Hk, Hv, Dk, Dv, chunk_size, code, 1,
+                                                                   need_states)
+    _lib.check(L.dllm_gdn_chunk_ws_fwd(
         q.data_ptr(), _lib.strides3(q), k.data_ptr(), _lib.strides3(k), v.data_ptr(), _lib.strides3(v),
         gg.data_ptr(), _lib.strides3(gg), bb.data_ptr(), _lib.strides3(bb), _lib.ptr(init), out.data_ptr(),
         _lib.ptr(states), B, T, Hk, Hv, Dk, Dv, chunk_size, code, int(bool(use_qk_l2norm_in_kernel)),
-        Dk ** -0.5, _lib.stream_handle(dev)), "dllm_gdn_chunk_fwd")
+        Dk ** -0.5, _lib.ptr(ws), nws, _lib.stream_handle(dev)), "dllm_gdn_chunk_fwd")
     _IMPL["last"], _IMPL["reason"] = "hip", ""
     return out, states
+
+
+def _scan_workspace(L, dev, B: int, T: int, Hk: int, Hv: int, Dk: int, Dv: int, chunk: int, code: int, streams: int,
+                    states: bool):
+    """Workspace of the prepared-tile path (few heads, bf16 128 x 128) and its bytes, from the stream's
+    caching allocator for this call; (None, 0) for shapes that path does not take."""
+    n = L.dllm_gdn_scan_workspace_bytes(B, T, Hk, Hv, Dk, Dv, chunk, code, streams, int(states))
+    return (torch.empty(n, dtype=torch.uint8, device=dev), n) if n > 0 else (None, 0)
 
 
 def _core(q, k, v, g, beta, *, chunk_size, initial_state, need_states):
@@ -245,7 +256,8 @@ def gdn_state_fork(raw0: torch.Tensor, rawt: torch.Tensor, conv_weight: torch.Te
     layer (B = 8, L = 2048, a head's columns over two workgroups) 381 vs 405 us. Without the
     states the fork is bound by its tile chain rather than by its stores, so the conv's arithmetic
     costs it more than the conv launch saves (the 16-layer stack's layers, B = 1, L = 2048: fork
-    258 vs 224 us, conv 19 vs 34 us)."""
+    258 vs 224 us, conv 19 vs 34 us). Few heads (at most 64 (sequence, head) pairs, ten tiles or more)
+    take the conv of every channel, then the prepared-tile path (csrc/gdn_scan.hip), bit-identical."""
     dev = _lib.require_device(raw0, rawt, conv_weight, beta0, betat, g0, gt, conv_bias)
     if raw0.shape != rawt.shape or raw0.dim() != 3:
         raise ValueError("raw0 and rawt must both be [B, L, conv_dim]")
@@ -293,8 +305,9 @@ def gdn_state_fork(raw0: torch.Tensor, rawt: torch.Tensor, conv_weight: torch.Te
                  and y0.data_ptr() % 16 == 0 and yt.data_ptr() % 16 == 0)
     vc_ok = (vconv_supported(Lb, K, Dk, Dv, block, code) and fault is None
              and all(t.data_ptr() % 16 == 0 for t in (r0, rt, y0, yt)))
-    if vconv is None:
-        vconv = vc_ok and states is not None
+    if vconv is None:  # few heads: the prepared-tile path on the conv of every channel is the faster one
+        vconv = (vc_ok and states is not None
+                 and Lb.dllm_gdn_scan_workspace_bytes(B, L, Hk, Hv, Dk, Dv, block, code, 2, 1) <= 0)
     elif vconv and not vc_ok:
         raise ValueError("vconv needs the pipelined fork kernel (bf16, Dk = Dv = 128, block dividing 32), a width-4 "
                          "conv, 16-byte aligned buffers and no fault")
@@ -325,12 +338,13 @@ def gdn_state_fork(raw0: torch.Tensor, rawt: torch.Tensor, conv_weight: torch.Te
         r0.data_ptr(), rt.data_ptr(), w.data_ptr(), _lib.ptr(bias), y0.data_ptr(), yt.data_ptr(),
         _lib.ptr(tails), B, L, Cd, K, block, code, wcode, cflags, sh), "dllm_conv_fork_fwd")
     if Lb.dllm_gdn_fused_fork_supported(Dk, block, code):
-        _lib.check(Lb.dllm_gdn_state_fork_fwd(
+        ws, nws = _scan_workspace(Lb, dev, B, L, Hk, Hv, Dk, Dv, block, code, 2, states is not None)
+        _lib.check(Lb.dllm_gdn_state_fork_ws_fwd(
             y0.data_ptr(), yt.data_ptr(), L * Cd, Cd, b0.data_ptr(), bt_.data_ptr(), gg0.data_ptr(), ggt.data_ptr(),
-            o0.data_ptr(), ot.data_ptr(), _lib.ptr(states), B, L, Hk, Hv, Dk, Dv, block, code, Dk ** -0.5, sh),
-            "dllm_gdn_state_fork_fwd")
+            o0.data_ptr(), ot.data_ptr(), _lib.ptr(states), B, L, Hk, Hv, Dk, Dv, block, code, Dk ** -0.5, _lib.ptr(ws),
+            nws, sh), "dllm_gdn_state_fork_fwd")
         path = Lb.dllm_gdn_state_fork_path(Dk, Dv, block, code)
-        _IMPL["last"], _IMPL["reason"] = "hip", _FORK_PATHS.get(path, "")
+        _IMPL["last"], _IMPL["reason"] = "hip", _FORK_PATHS.get(path, "") + (", tiles prepared ahead" if nws else "")
     else:
         # two-pass fork on the same HIP core: clean pass with states, then the B*nb noised rows
         # relaunched from the shifted states (reference blockdiff.py:160-176)
@@ -559,11 +573,15 @@ class StateForkPlan:
         # and the states are kept
         ok = (vconv_supported(self._lib, K, head_k_dim, head_v_dim, block, self.code)
               and raw0.data_ptr() % 16 == 0 and rawt.data_ptr() % 16 == 0)
+        nws = self._lib.dllm_gdn_scan_workspace_bytes(B, L, num_k_heads, num_v_heads, head_k_dim, head_v_dim, block,
+                                                      self.code, 2, int(need_states))
         if vconv is None:
-            vconv = ok and need_states
+            vconv = ok and need_states and nws <= 0
         elif vconv and not ok:
             raise ValueError("vconv needs the pipelined fork kernel (bf16, Dk = Dv = 128) and a width-4 conv")
         self.vconv = bool(vconv)
+        # the prepared-tile path's workspace (few heads)
+        self.ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 and not vconv else None
 
     def run_conv(self, stream=None):
         B, L, Cd, Hk, Hv, Dk, Dv, block = self.dims
@@ -591,10 +609,11 @@ class StateForkPlan:
                 self.ot.data_ptr(), _lib.ptr(self.states), B, L, Hk, Hv, Dk, Dv, block, self.code, Dk ** -0.5, 0,
                 L // block, sh), "dllm_gdn_state_fork_vconv_range_fwd")
             return
-        _lib.check(self._lib.dllm_gdn_state_fork_fwd(
+        _lib.check(self._lib.dllm_gdn_state_fork_ws_fwd(
             self.y0.data_ptr(), self.yt.data_ptr(), L * Cd, Cd, self.beta0.data_ptr(), self.betat.data_ptr(),
             self.g0.data_ptr(), self.gt.data_ptr(), self.o0.data_ptr(), self.ot.data_ptr(), _lib.ptr(self.states),
-            B, L, Hk, Hv, Dk, Dv, block, self.code, Dk ** -0.5, sh), "dllm_gdn_state_fork_fwd")
+            B, L, Hk, Hv, Dk, Dv, block, self.code, Dk ** -0.5, _lib.ptr(self.ws),
+            0 if self.ws is None else self.ws.numel(), sh), "dllm_gdn_state_fork_fwd")
 
     def run(self, stream=None):
         self.run_conv(stream)

@@ -49,6 +49,23 @@ int dllm_gdn_chunk_fwd(const void* q, const int64_t* q_strides, const void* k, c
                        int chunk, int dtype, int use_qk_l2norm, float scale, void* stream);
 
 /*
+ * dllm_gdn_chunk_fwd with a caller's workspace (256-byte aligned, dllm_gdn_scan_workspace_bytes(..,
+ * 1, states) bytes; null: none): bf16 heads of 128 x 128 with at most 64 (sequence, head) pairs and at
+ * least ten tiles then run in two launches, every tile's preparation at once and the recurrence alone after
+ * it, instead of the pipelined kernel. Results are the same bits. dllm_gdn_scan_workspace_bytes returns
+ * 0 for shapes this path does not take (the workspace is then ignored); streams: 1 for the chunked
+ * rule, 2 for the state fork (dllm_gdn_state_fork_ws_fwd); states: nonzero when the states are wanted. No counterpart in the reference.
+ */
+long long dllm_gdn_scan_workspace_bytes(int B, int T, int Hk, int Hv, int Dk, int Dv, int chunk, int dtype, int streams,
+                                        int states);
+int dllm_gdn_chunk_ws_fwd(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
+                          const void* v, const int64_t* v_strides, const float* g, const int64_t* g_strides,
+                          const float* beta, const int64_t* beta_strides, const float* initial_state,
+                          void* out, float* states, int B, int T, int Hk, int Hv, int Dk, int Dv,
+                          int chunk, int dtype, int use_qk_l2norm, float scale, void* workspace,
+                          long long workspace_bytes, void* stream);
+
+/*
  * 1 if the fused state-fork kernel handles (Dk, block, dtype): block divides 32, Dk <= 128, and
  * Dk <= 64 for float32. Otherwise callers run the two-pass fork (dllm_gdn_chunk_fwd on the clean
  * stream with states, then again on the B*nb noised rows with initial states), as the reference
@@ -81,6 +98,16 @@ int dllm_gdn_state_fork_fwd(const void* qkv0, const void* qkvt, int64_t qkv_stri
                             const float* beta0, const float* betat, const float* g0, const float* gt,
                             void* out0, void* outt, float* states, int B, int L, int Hk, int Hv, int Dk,
                             int Dv, int block, int dtype, float scale, void* stream);
+
+/*
+ * dllm_gdn_state_fork_fwd with a caller's workspace (dllm_gdn_scan_workspace_bytes(.., 2, states)
+ * bytes), as dllm_gdn_chunk_ws_fwd takes one. Results are the same bits with and without it.
+ */
+int dllm_gdn_state_fork_ws_fwd(const void* qkv0, const void* qkvt, int64_t qkv_stride_b, int64_t qkv_stride_t,
+                               const float* beta0, const float* betat, const float* g0, const float* gt,
+                               void* out0, void* outt, float* states, int B, int L, int Hk, int Hv, int Dk,
+                               int Dv, int block, int dtype, float scale, void* workspace,
+                               long long workspace_bytes, void* stream);
 
 /*
  * The same op over blocks [block_begin, block_end) of every sequence, for callers that overlap the
