@@ -1046,6 +1046,241 @@ static int launch_attn_sp(const AttnArgs& a, hipStream_t st) {
   return DLLM_OK;
 }
 
+// ---------------------------------------------------------------------------------------------
+// fp32, d == D in {32, 64, 128, 256} with 16-byte rows: one workgroup of four waves per 32-query tile and
+// head, the waves taking the tile's key tiles in turn (wave w the tiles w, w + 4, ..), each with its own
+// running max, sum and O^T, merged through LDS at the end. Bound by the fp32 matrix cores: a key tile is
+// 32 D / 32 32x32x2 products of 64 clocks (16k clocks at D = 256) against 64 KB of K and V, so the
+// operands come straight from L2 as fragments (K 16 bytes per lane, V^T 128 bytes per key and
+// instruction), a few slices ahead of their products, with no staging and no barrier in the loop; only Q
+// sits in LDS. Four 32-query tiles per workgroup with K/V staged for them, the kernel for the other layouts,
+// leaves most SIMDs idle at short lengths. B = 1, 24 / 4 heads of 256, us there -> here: L = 256 133 -> 42,
+// L = 32 36 -> 15, L = 2048 1203 -> 1100 (103 TFLOP/s over the visible tiles); 32 rows of block-causal
+// queries against 4128 keys 1190 -> 284. Two slices ahead at D = 256: one 40 / 16 / 1023 / 388, three with
+// 512 registers a lane 42 / 16 / 954 / 275 (178 -> 189 at two sequences of 512).
+// ---------------------------------------------------------------------------------------------
+template <int D, bool BC>
+__global__ __launch_bounds__(256, 2) void bd_attn_f32_kernel(AttnArgs a) {
+  using F = Frag<false>;
+  constexpr int DT = D / 32, NW = 4;
+  constexpr int ROW = D + 4;                 // floats per staged row (Q, then O on its way between waves)
+  constexpr int NR = DT < 3 ? DT : DT == 8 ? 2 : 3;  // operand slices in flight ahead of their products
+  __shared__ __attribute__((aligned(16))) float smem[2 * 32 * ROW + NW * 64];
+  float* const ml = smem + 2 * 32 * ROW;     // [wave][max 32 | sum 32]
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, h = lane >> 5, l32 = lane & 31;
+  const int L = a.L, C = a.C;
+  const int Lq = BC ? a.M : L;
+  const int Lk = BC ? a.N : L;
+  const int qa = BC ? a.q0 : 0;
+  const int ntq = (Lq + 31) >> 5;
+  const int rep = a.Hq / a.Hkv;
+
+  // work unit: longest first (query tile descending), then half, batch, KV head, query head in group
+  constexpr int NH = BC ? 1 : 2;
+  const int lin = attn_unit(blockIdx.x, gridDim.x, NH * rep);
+  const int per_g = NH * a.B * a.Hkv * rep;
+  const int r0 = (ntq - 1 - lin / per_g) * 32, r1 = min(Lq, r0 + 32);
+  int rem = lin % per_g;
+  const int qh = BC ? 1 : rem % 2;
+  rem /= NH;
+  const int hr = rem % rep;
+  rem /= rep;
+  const int hkv = rem % a.Hkv;
+  const int b = rem / a.Hkv;
+  const int hq = hkv * rep + hr;
+  const int qb0 = (qa + r0) / C, qb1 = (qa + r1 - 1) / C;
+  int lo0, hi0, hi1;  // keys of half 0 (x_t) [lo0, hi0) and of half 1 (x_0) [0, hi1) that some query sees
+  if (qh == 1) {
+    lo0 = hi0 = 0;
+    hi1 = min(Lk, (qb1 + 1) * C);
+  } else {
+    lo0 = a.leak ? 0 : qb0 * C;
+    hi0 = min(L, (qb1 + 1) * C);
+    hi1 = min(L, qb1 * C);
+  }
+  const int t0lo = lo0 >> 5, n0 = hi0 > lo0 ? ((hi0 + 31) >> 5) - t0lo : 0;
+  const int n1 = hi1 > 0 ? (hi1 + 31) >> 5 : 0;
+  const int ntiles = n0 + n1;  // x_0 tiles first, then x_t tiles
+
+  const float* const qbase = (const float*)a.q + b * a.q_sb + (long long)hq * a.q_sh;
+  const float* const kbase = (const float*)a.k + b * a.k_sb + (long long)hkv * a.k_sh;
+  const float* const vbase = (const float*)a.v + b * a.v_sb + (long long)hkv * a.v_sh;
+#pragma unroll
+  for (int i = 0; i < DT; ++i) {  // Q rows (past the last: a valid row, never stored)
+    const int e = i * 256 + tid, row = e / (D / 4), c = (e % (D / 4)) * 4;
+    *(f32x4*)(smem + row * ROW + c) =
+        *(const f32x4*)(qbase + (long long)((BC ? 0 : qh * L) + min(r0 + row, Lq - 1)) * a.q_st + c);
+  }
+  __syncthreads();
+
+  // keys visible to this lane's query in each half
+  const int qi = r0 + l32, qbl = (qa + qi) / C;
+  int vlo0 = 0, vhi0 = 0, vhi1;
+  if (qh == 1) {
+    vhi1 = min(Lk, (qbl + 1) * C);
+  } else {
+    vlo0 = a.leak ? 0 : qbl * C;
+    vhi0 = min(Lk, (qbl + 1) * C);
+    vhi1 = min(Lk, qbl * C);
+  }
+  f32x16 O[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) O[t] = zero16();
+  float mrow = -1e30f, lrow = 0.f;  // running max (log2 units) and sum of this lane's query
+
+  for (int n = wave; n < ntiles; n += NW) {
+    const int kh = n < n1 ? 1 : 0;
+    const int j0 = (n < n1 ? n : t0lo + n - n1) * 32;
+    const long long tile_row = (long long)((BC ? 0 : kh * L) + j0);
+    const int past = Lk - 1 - j0;  // rows past the last key load it; their scores are masked
+    const float* const kp = kbase + tile_row * a.k_st + (long long)min(l32, past) * a.k_st + 4 * h;
+    F kf[NR];
+    auto load_k = [&](int s, F& f) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const f32x4 r = *(const f32x4*)(kp + 32 * s + 8 * m);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f.v[4 * m + e] = r[e];
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < NR; ++s) load_k(s, kf[s]);
+    f32x16 st = zero16();
+#pragma unroll
+    for (int s = 0; s < DT; ++s) {
+      F qf;
+      lds_frag(smem + l32 * ROW + 32 * s, h, qf);
+      mma32(st, kf[s % NR], qf);
+      if (s + NR < DT) load_k(s + NR, kf[s % NR]);
+      __builtin_amdgcn_sched_barrier(0);  // one slice's operands at a time: registers
+    }
+    // V^T fragments: column 32 t + l32 of the keys in rho order
+    const float* const vp = vbase + tile_row * a.v_st;
+    unsigned voff[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) voff[v] = (unsigned)(min(rho(v, h), past) * a.v_st + l32);
+    F vf[NR];
+    auto load_v = [&](int t, F& f) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) f.v[v] = (vp + 32 * t)[voff[v]];
+    };
+#pragma unroll
+    for (int t = 0; t < NR; ++t) load_v(t, vf[t]);
+    const int lo = kh ? 0 : vlo0, hi = kh ? vhi1 : vhi0;
+    float mx = -INFINITY;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const int kj = j0 + rho(v, h);
+      st[v] = (kj >= lo && kj < hi) ? st[v] * a.scale_log2e : -INFINITY;
+      mx = fmaxf(mx, st[v]);
+    }
+    mx = halves_max(mx);
+    // lazy rescale (see bd_attn_kernel)
+    constexpr float RESCALE_LOG2 = 8.f;
+    if (__builtin_amdgcn_ballot_w64(mx > mrow + RESCALE_LOG2) != 0) {
+      const float mnew = fmaxf(mrow, mx);
+      const float alpha = __builtin_amdgcn_exp2f(mrow - mnew);
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) O[t][v] *= alpha;
+      lrow *= alpha;
+      mrow = mnew;
+    }
+    F pf;
+    float ps = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      pf.v[v] = __builtin_amdgcn_exp2f(st[v] - mrow);
+      ps += pf.v[v];
+    }
+    lrow += halves_sum(ps);
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {  // O^T += V^T P^T
+      mma32(O[t], vf[t % NR], pf);
+      if (t + NR < DT) load_v(t + NR, vf[t % NR]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+
+  // merge: every wave to the common maximum, then 1 -> 0 and 3 -> 2, then 2 -> 0
+  if (h == 0) {
+    ml[64 * wave + l32] = mrow;
+    ml[64 * wave + 32 + l32] = lrow;
+  }
+  __syncthreads();  // also: every wave is done with Q
+  float m = ml[l32];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) m = fmaxf(m, ml[64 * w + l32]);
+  float l = 0.f;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) l += ml[64 * w + 32 + l32] * __builtin_amdgcn_exp2f(ml[64 * w + l32] - m);
+  const float wsc = __builtin_amdgcn_exp2f(mrow - m);
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) O[t][v] *= wsc;
+  auto put = [&](float* buf) {
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = O[t][4 * q + e];
+        *(f32x4*)(buf + l32 * ROW + 32 * t + 8 * q + 4 * h) = x;
+      }
+  };
+  auto add = [&](const float* buf) {
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const f32x4 x = *(const f32x4*)(buf + l32 * ROW + 32 * t + 8 * q + 4 * h);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) O[t][4 * q + e] += x[e];
+      }
+  };
+  float* const buf1 = smem + 32 * ROW;
+  if (wave == 1) put(smem);
+  if (wave == 3) put(buf1);
+  __syncthreads();
+  if (wave == 0) add(smem);
+  if (wave == 2) add(buf1);
+  __syncthreads();
+  if (wave == 2) put(buf1);
+  __syncthreads();
+  if (wave == 0) {
+    add(buf1);
+    const float inv = 1.f / l;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) O[t][v] *= inv;
+    put(smem);
+  }
+  __syncthreads();
+  const long long orow = BC ? (long long)b * Lq + r0 : (long long)b * 2 * L + qh * L + r0;
+#pragma unroll
+  for (int i = 0; i < DT; ++i) {
+    const int e = i * 256 + tid, row = e / (D / 4), c = (e % (D / 4)) * 4;
+    if (r0 + row < Lq) *(f32x4*)((float*)a.out + ((orow + row) * a.Hq + hq) * D + c) = *(const f32x4*)(smem + row * ROW + c);
+  }
+}
+
+template <int D, bool BC>
+static int launch_attn_f32(const AttnArgs& a, hipStream_t st) {
+  const int ntq = ((BC ? a.M : a.L) + 31) / 32;
+  const long long nblk = (long long)ntq * (BC ? 1 : 2) * a.B * a.Hq;
+  if (nblk > 0x7fffffff) return fail(DLLM_EUNSUPPORTED, "attention: grid too large");
+  bd_attn_f32_kernel<D, BC><<<dim3((unsigned)nblk), dim3(256), 0, st>>>(a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return fail(DLLM_ELAUNCH, "attention launch: %s", hipGetErrorString(e));
+  return DLLM_OK;
+}
+
 static bool fits32(long long x) { return x >= -2147483647LL && x <= 2147483647LL; }
 
 // shared by both entry points: vectorisation check and kernel choice
@@ -1082,6 +1317,15 @@ static int dispatch_attn(AttnArgs& a, const int64_t* const sts[3], int dtype, hi
   }
   if (direct_only) return fail(DLLM_EUNSUPPORTED, "attention: the gated form is bf16 only");
   if (dtype == DT_F32) {
+    // the key-split kernel: whole 16-byte rows, and a tile's V rows within 32-bit element offsets
+    if (vec && ((uintptr_t)a.out % 16) == 0 && a.v_st >= 0 && a.v_st < (1 << 25)) {
+      switch (dw) {
+        case 32: return launch_attn_f32<32, BC>(a, st);
+        case 64: return launch_attn_f32<64, BC>(a, st);
+        case 128: return launch_attn_f32<128, BC>(a, st);
+        default: return launch_attn_f32<256, BC>(a, st);
+      }
+    }
     switch (dw) {
       case 32: return launch_attn<32, false, BC>(a, st);
       case 64: return launch_attn<64, false, BC>(a, st);

@@ -130,3 +130,24 @@ def test_empty_queries_give_empty_outputs(dev):
     k = torch.randn(2, 96, 2, 64, device=dev, dtype=torch.bfloat16)
     assert attention.block_causal_attention(q, k, k, block=32, q_offset=64).shape == (2, 0, 4, 64)
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("B,L,Hq,Hkv,d,block,leak,scale", [
+    (1, 8, 2, 1, 256, 8, False, None),     # one ragged key tile per half: three waves have none
+    (2, 72, 6, 2, 256, 24, False, None),   # last tile of 8 rows, as many key tiles as waves and fewer
+    (1, 264, 4, 2, 256, 8, True, None),    # more key tiles than waves, the x_t prefix visible too
+    (1, 160, 4, 4, 128, 32, False, -0.05),  # negative scale
+    (1, 136, 3, 1, 64, 8, False, 0.0),
+    (2, 200, 4, 2, 32, 40, False, None),
+])
+@pytest.mark.parametrize("pad", [0, 4, 2])  # V (and K) row padding: 2 floats is no whole 16 bytes
+def test_fp32_key_split_matches_oracle(dev, B, L, Hq, Hkv, d, block, leak, scale, pad):
+    """fp32 with 16-byte rows: the key tiles are shared by a workgroup's waves and merged; rows of other
+    strides take the staged kernel. Both within the fp32 bar of the oracle."""
+    q, k, v = _inputs(B, L, Hq, Hkv, d, torch.float32, seed=L + d + block)
+    buf = [torch.zeros(B, 2 * L, Hkv, d + pad, device=dev) for _ in range(2)]
+    kd, vd = buf[0][..., :d].copy_(k), buf[1][..., :d].copy_(v)
+    got = attention.bd_attention(q.to(dev), kd, vd, block=block, scale=scale, leak_xt_prefix=leak)
+    torch.cuda.synchronize()
+    ref = attn_ref.bd_attention(q, k, v, block=block, scale=scale, leak_xt_prefix=leak)
+    _check(got, ref, torch.float32, f"L{L} d{d} block{block} pad{pad}")
