@@ -37,7 +37,8 @@ def last_impl():
 
 
 def _fp32c(t: torch.Tensor) -> torch.Tensor:
-    return t.to(torch.float32).contiguous()
+    # the two no-op conversions of a tensor that is float32 and contiguous already cost 1.1 us, the look 0.3
+    return t if t.dtype is torch.float32 and t.is_contiguous() else t.to(torch.float32).contiguous()
 
 
 def _lastdim_contig(t: torch.Tensor) -> torch.Tensor:
