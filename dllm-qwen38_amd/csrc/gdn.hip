@@ -1526,6 +1526,16 @@ extern "C" long long dllm_gdn_scan_workspace_bytes(int B, int T, int Hk, int Hv,
   return gdn_scan_workspace(B, T, Hk, Hv, chunk, streams, states != 0, nullptr);
 }
 
+// The fp32 fork by prepared tiles (gdn_scan_f32.hip): square heads of 64 or 128, blocks that divide the
+// 32-row tile, from one block on. Heads of 64 have a one-launch kernel, which takes over where a workgroup per
+// head fills the chip (L = 256: 128 heads 134 vs 95 us, 192 heads 139 vs 147; two blocks of four heads 36 vs 36).
+extern "C" long long dllm_gdn_fork_f32_workspace_bytes(int B, int L, int Hk, int Hv, int Dk, int Dv, int block, int states) {
+  if (B <= 0 || L <= 0 || Hk <= 0 || Hv <= 0 || block <= 0 || Hv % Hk || L % block || 32 % block) return 0;
+  if (Dk != Dv || (Dk != 64 && Dk != 128)) return 0;
+  if (Dk == 64 && (long long)B * Hv > 128) return 0;
+  return gdn_fork32_workspace(B, L, Hk, Hv, Dk, block, states != 0, nullptr);
+}
+
 // Whether the prepared-tile path runs: shape (need > 0) and a workspace for it. A workspace that is too
 // small or misaligned is an error (sets *rc).
 static bool scan_taken(long long need, void* workspace, long long workspace_bytes, int* rc) {
@@ -1636,7 +1646,9 @@ static int state_fork(const void* qkv0, const void* qkvt, int64_t qkv_stride_b, 
     return fail(DLLM_EINVAL, "gdn fork: bad sizes");
   if (L % block) return fail(DLLM_EINVAL, "L=%d is not a multiple of block=%d", L, block);
   if (Hv % Hk) return fail(DLLM_EINVAL, "gdn fork: Hv=%d is not a multiple of Hk=%d", Hv, Hk);
-  if (!dllm_gdn_fused_fork_supported(Dk, block, dtype))
+  const long long need32 =
+      dtype == DT_F32 && workspace ? dllm_gdn_fork_f32_workspace_bytes(B, L, Hk, Hv, Dk, Dv, block, states != nullptr) : 0;
+  if (need32 == 0 && !dllm_gdn_fused_fork_supported(Dk, block, dtype))
     return fail(DLLM_EUNSUPPORTED, "gdn fork: fused fork unsupported for Dk=%d block=%d dtype=%d", Dk, block, dtype);
   if (!fits_i32((long long)L * qkv_stride_t) || !fits_i32((long long)L * Hv))
     return fail(DLLM_EUNSUPPORTED, "gdn fork: per-sequence extent exceeds 32-bit element offsets");
@@ -1716,6 +1728,11 @@ static int state_fork(const void* qkv0, const void* qkvt, int64_t qkv_stride_b, 
                             workspace_bytes, &rc))
       return rc == DLLM_OK ? gdn_scan_launch(a, 2, workspace, (hipStream_t)stream) : rc;
     return launch_fork_pipe<2>(a, (hipStream_t)stream);
+  }
+  if (need32 > 0 && whole && a.vec_qk && a.vec_v) {
+    int rc;
+    if (scan_taken(need32, workspace, workspace_bytes, &rc))
+      return rc == DLLM_OK ? gdn_fork32_launch(a, workspace, (hipStream_t)stream) : rc;
   }
   if (!whole) return fail(DLLM_EUNSUPPORTED, "gdn fork: block ranges need the pipelined kernel (bf16, Dk = Dv = 128)");
   return dispatch_gdn(a, dtype, true, (hipStream_t)stream);

@@ -164,6 +164,14 @@ __device__ __forceinline__ void store_snapshot_slice(float* p0, const f32x16& s)
   store_snapshot<3584>(p1, s[15]);
 }
 
+// Touch one 128-byte line per lane, so that the tile's operands wait in this XCD's L2 (no register
+// result: the four bytes per lane land in a spare LDS area).
+__device__ __forceinline__ void scan_touch(const void* src, const void* lds_base) {
+  typedef const __attribute__((address_space(3))) void* lds_cptr;
+  const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_cptr)lds_base);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
+}
+
 // Launch arguments of one stream's whole sequence are filled by the entry points in gdn.hip; the
 // prepared-tile path (gdn_scan.hip) takes the same arguments.
 //
@@ -171,5 +179,8 @@ __device__ __forceinline__ void store_snapshot_slice(float* p0, const f32x16& s)
 long long gdn_scan_workspace(int B, int T, int Hk, int Hv, int sub, int streams, bool states,
                              int* tiles_per_range);
 int gdn_scan_launch(const GdnArgs& a, int streams, void* workspace, hipStream_t st);
+// The same for the fp32 state fork (gdn_scan_f32.hip): D = Dk = Dv, 64 or 128.
+long long gdn_fork32_workspace(int B, int L, int Hk, int Hv, int D, int block, bool states, int* tiles_per_range);
+int gdn_fork32_launch(const GdnArgs& a, void* workspace, hipStream_t st);
 
 }  // namespace dllm

@@ -233,14 +233,6 @@ struct ScanSmem {
   static constexpr int TOTAL = O_SN + 2 * SN;
 };
 
-// Touch one 128-byte line per lane, so that the tile's operands wait in this XCD's L2 (no register
-// result: the four bytes per lane land in a spare LDS area).
-__device__ __forceinline__ void scan_touch(const void* src, const void* lds_base) {
-  typedef const __attribute__((address_space(3))) void* lds_cptr;
-  const unsigned m0 = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(lds_cptr)lds_base);
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(src), "s"(m0) : "memory", "m0");
-}
-
 // One workgroup per (sequence, value head, 32 value columns), its waves split by role so that the state's
 // chain is all that wave 0 does:
 //   wave 0     the clean state, in accumulators: per tile it publishes the state before the tile (as B

@@ -34,6 +34,7 @@ _SIGNATURES = {
         _c_fp, _c_void_p, _c_fp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
         _c_float, _c_void_p]),
     "dllm_gdn_scan_workspace_bytes": (_c_i64, [_c_int] * 10),
+    "dllm_gdn_fork_f32_workspace_bytes": (_c_i64, [_c_int] * 8),
     "dllm_gdn_chunk_ws_fwd": (_c_int, [
         _c_void_p, _c_i64p, _c_void_p, _c_i64p, _c_void_p, _c_i64p, _c_fp, _c_i64p, _c_void_p, _c_i64p,
         _c_fp, _c_void_p, _c_fp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,

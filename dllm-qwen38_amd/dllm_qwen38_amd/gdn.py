@@ -338,14 +338,20 @@ def gdn_state_fork(raw0: torch.Tensor, rawt: torch.Tensor, conv_weight: torch.Te
     _lib.check(Lb.dllm_conv_fork_fwd(
         r0.data_ptr(), rt.data_ptr(), w.data_ptr(), _lib.ptr(bias), y0.data_ptr(), yt.data_ptr(),
         _lib.ptr(tails), B, L, Cd, K, block, code, wcode, cflags, sh), "dllm_conv_fork_fwd")
-    if Lb.dllm_gdn_fused_fork_supported(Dk, block, code):
+    if dt == torch.float32:
+        # prepared tiles in fp32, on the 16-byte rows of the conv outputs
+        nws = (Lb.dllm_gdn_fork_f32_workspace_bytes(B, L, Hk, Hv, Dk, Dv, block, int(states is not None))
+               if y0.data_ptr() % 16 == 0 and yt.data_ptr() % 16 == 0 else 0)
+        ws = torch.empty(nws, dtype=torch.uint8, device=dev) if nws > 0 else None
+    else:
         ws, nws = _scan_workspace(Lb, dev, B, L, Hk, Hv, Dk, Dv, block, code, 2, states is not None)
+    if nws > 0 or Lb.dllm_gdn_fused_fork_supported(Dk, block, code):
         _lib.check(Lb.dllm_gdn_state_fork_ws_fwd(
             y0.data_ptr(), yt.data_ptr(), L * Cd, Cd, b0.data_ptr(), bt_.data_ptr(), gg0.data_ptr(), ggt.data_ptr(),
             o0.data_ptr(), ot.data_ptr(), _lib.ptr(states), B, L, Hk, Hv, Dk, Dv, block, code, Dk ** -0.5, _lib.ptr(ws),
             nws, sh), "dllm_gdn_state_fork_fwd")
         path = Lb.dllm_gdn_state_fork_path(Dk, Dv, block, code)
-        _IMPL["last"], _IMPL["reason"] = "hip", _FORK_PATHS.get(path, "") + (", tiles prepared ahead" if nws else "")
+        _IMPL["last"], _IMPL["reason"] = "hip", _FORK_PATHS[path] + (", tiles prepared ahead" if nws else "")
     else:
         # two-pass fork on the same HIP core: clean pass with states, then the B*nb noised rows
         # relaunched from the shifted states (reference blockdiff.py:160-176)
@@ -369,7 +375,7 @@ def gdn_state_fork(raw0: torch.Tensor, rawt: torch.Tensor, conv_weight: torch.Te
 
 
 # kernel names reported through last_impl() for the fused fork (dllm_gdn_state_fork_path)
-_FORK_PATHS = {2: "pipelined fork kernel", 1: "fused fork kernel"}
+_FORK_PATHS = {2: "pipelined fork kernel", 1: "fused fork kernel", 0: "fork of prepared tiles"}
 
 _CUS: dict = {}
 _SIDE = threading.local()
@@ -574,8 +580,12 @@ class StateForkPlan:
         # and the states are kept
         ok = (vconv_supported(self._lib, K, head_k_dim, head_v_dim, block, self.code)
               and raw0.data_ptr() % 16 == 0 and rawt.data_ptr() % 16 == 0)
-        nws = self._lib.dllm_gdn_scan_workspace_bytes(B, L, num_k_heads, num_v_heads, head_k_dim, head_v_dim, block,
-                                                      self.code, 2, int(need_states))
+        if dt == torch.float32:
+            nws = self._lib.dllm_gdn_fork_f32_workspace_bytes(B, L, num_k_heads, num_v_heads, head_k_dim, head_v_dim,
+                                                              block, int(need_states))
+        else:
+            nws = self._lib.dllm_gdn_scan_workspace_bytes(B, L, num_k_heads, num_v_heads, head_k_dim, head_v_dim, block,
+                                                          self.code, 2, int(need_states))
         if vconv is None:
             vconv = ok and need_states and nws <= 0
         elif vconv and not ok:

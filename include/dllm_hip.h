@@ -101,8 +101,12 @@ int dllm_gdn_state_fork_fwd(const void* qkv0, const void* qkvt, int64_t qkv_stri
 
 /*
  * dllm_gdn_state_fork_fwd with a caller's workspace (dllm_gdn_scan_workspace_bytes(.., 2, states)
- * bytes), as dllm_gdn_chunk_ws_fwd takes one. Results are the same bits with and without it.
+ * bytes), as dllm_gdn_chunk_ws_fwd takes one. In bf16 the results are the same bits with and without it.
+ * In fp32 the workspace (dllm_gdn_fork_f32_workspace_bytes bytes, 0 for shapes that do not take one: square
+ * heads of 64 or 128, 16-byte rows, a block dividing 32) prepares every tile at once as well, and
+ * serves the 128 x 128 heads that dllm_gdn_fused_fork_supported does not; sums run in another order.
  */
+long long dllm_gdn_fork_f32_workspace_bytes(int B, int L, int Hk, int Hv, int Dk, int Dv, int block, int states);
 int dllm_gdn_state_fork_ws_fwd(const void* qkv0, const void* qkvt, int64_t qkv_stride_b, int64_t qkv_stride_t,
                                const float* beta0, const float* betat, const float* g0, const float* gt,
                                void* out0, void* outt, float* states, int B, int L, int Hk, int Hv, int Dk,
