@@ -27,12 +27,14 @@ template <typename TX, typename TW, int K, int VEC, int BLK>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BLK > 0 ? 5 : 1, BLK > 0 ? 5 : 8))) void conv_fork_kernel(
     const TX* __restrict__ raw0, const TX* __restrict__ rawt, const TW* __restrict__ w,
     const TW* __restrict__ bias, TX* __restrict__ y0, TX* __restrict__ yt, TX* __restrict__ tails,
-    int L, int Cd, int block, int cold_noised, int kb_off, int cy) {
+    int L, int Cd, int block, int cold_noised, int kb_off, int cy, int seg) {
   const int cg = blockIdx.x * blockDim.x + threadIdx.x;  // channel group
   const int c0 = cg * VEC;
   if (c0 >= cy) return;  // channels [cy, Cd): not this launch's (their conv runs elsewhere)
-  if (BLK > 0) block = BLK;
-  const int kblk = blockIdx.y + kb_off;  // the launch covers blocks [kb_off, kb_off + gridDim.y)
+  if (BLK > 0) block = seg = BLK;
+  // rows [s0, s0 + seg) of a block; the launch covers blocks from kb_off, block / seg segments each
+  const int nseg = BLK > 0 ? 1 : block / seg;
+  const int kblk = blockIdx.y / nseg + kb_off, s0 = (blockIdx.y % nseg) * seg;
   const int b = blockIdx.z;
   const int nb = L / block;
 
@@ -51,7 +53,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BLK > 0 ? 5
   TX tl[VEC * (K - 1)];  // this thread's conv tails, channel-major: VEC*(K-1) consecutive elements
 #pragma unroll
   for (int j = 0; j < K - 1; ++j) {
-    const int p = fork_prefix_pos(kblk, j, block, K);
+    const int p = s0 ? kblk * block + s0 - (K - 1) + j : fork_prefix_pos(kblk, j, block, K);
     TX xs[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; ++e) xs[e] = from_f32<TX>(0.f);
@@ -66,8 +68,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BLK > 0 ? 5
       h0[j][e] = round_through<TW>(to_f32(xs[e]));
       ht[j][e] = cold_noised ? 0.f : h0[j][e];
     }
+    if (s0) {  // inside the block (seg >= K - 1): the noised stream's own rows
+      const TX* src = rawt + row_base + (long long)p * Cd + c0;
+#pragma unroll
+      for (int e = 0; e < VEC; ++e) ht[j][e] = round_through<TW>(to_f32(src[e]));
+    }
   }
-  if (tails) {
+  if (tails && s0 == 0) {
     TX* dst = tails + ((long long)fork_row(b, kblk, nb) * Cd + c0) * (K - 1);
     constexpr int TN = VEC * (K - 1);
     // widest store dividing the run: the run starts at element c0 * (K - 1), c0 a multiple of VEC
@@ -93,17 +100,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(BLK > 0 ? 5
   // computed, so each thread keeps 2*RG row loads in flight
   constexpr int RG = 4;
   const long long base = row_base + (long long)(kblk * block) * Cd + c0;
-  for (int r0 = 0; r0 < block; r0 += RG) {
+  for (int r0 = s0; r0 < s0 + seg; r0 += RG) {
     VecN<TX, VEC> x0v[RG], xtv[RG];
 #pragma unroll
     for (int q = 0; q < RG; ++q) {
-      const int r = min(r0 + q, block - 1);  // a ragged last group reloads the last row, unused
+      const int r = min(r0 + q, s0 + seg - 1);  // a ragged last group reloads the last row, unused
       x0v[q] = *(const VecN<TX, VEC>*)(raw0 + base + (long long)r * Cd);
       xtv[q] = *(const VecN<TX, VEC>*)(rawt + base + (long long)r * Cd);
     }
 #pragma unroll
     for (int q = 0; q < RG; ++q) {
-      if (r0 + q >= block) break;
+      if (r0 + q >= s0 + seg) break;
       const TX* x0 = x0v[q].v;
       const TX* xt = xtv[q].v;
       VecN<TX, VEC> o0v, otv;
@@ -166,6 +173,8 @@ __global__ __launch_bounds__(256) void conv_generic_kernel(
   }
 }
 
+constexpr int CONV_WGS = 512;
+
 template <typename TX, typename TW>
 static int launch_fork(const void* raw0, const void* rawt, const void* w, const void* bias, void* y0,
                        void* yt, void* tails, int B, int L, int Cd, int K, int block, int cold, int kb0,
@@ -177,39 +186,48 @@ static int launch_fork(const void* raw0, const void* rawt, const void* w, const 
                       ((uintptr_t)tails % 16 == 0);  // tails rows of VEC*(K-1) elements are 16-byte multiples
   bool done = false;
   if constexpr (V == 8) {
-    if (K == 4 && vec_ok && block == 32) {
+    if (K == 4 && vec_ok && block == 32 && (long long)((cy / 4 + 255) / 256) * nb * B >= 128) {
+      // (fewer blocks than that: split rows below, conv_dim 10240, L = 256 11.8 -> 9.9 us, L = 64 9.6 -> 6.1)
       // 8-byte channel groups at five resident waves per SIMD: at the 27B-class shape (B = 4,
       // L = 4096, conv_dim = 10240) the 20480 waves are exactly four rounds of the chip's slots
       const int groups = cy / 4;
       dim3 grid((groups + 255) / 256, nb, B);
       conv_fork_kernel<TX, TW, 4, 4, 32><<<grid, 256, 0, st>>>(
           (const TX*)raw0, (const TX*)rawt, (const TW*)w, (const TW*)bias, (TX*)y0, (TX*)yt, (TX*)tails, L,
-          Cd, block, cold, kb0, cy);
+          Cd, block, cold, kb0, cy, block);
       done = true;
     }
   }
   if (done) {
   } else if (K == 4 && vec_ok) {
     const int groups = cy / V;
-    dim3 grid((groups + 255) / 256, nb, B);
+    // One thread walks a block's rows four at a time, waiting for memory each time: with few blocks the rows
+    // go to up to block / 4 threads (which read the three rows before theirs again), while the launch
+    // has under CONV_WGS workgroups (fp32, conv_dim 10240: L = 256 25.4 -> 11.0 us, L = 512 27.6 -> 17.1; under 1024
+    // workgroups B = 2, L = 512 takes 31.2 for 28.9, unsplit 33.3)
+    int seg = block;
+    while (seg % 2 == 0 && seg > 4 && (long long)((groups + 255) / 256) * nb * B * (block / seg) < CONV_WGS &&
+           (long long)nb * (block / seg) * 2 <= 65535)
+      seg /= 2;
+    dim3 grid((groups + 255) / 256, nb * (block / seg), B);
     conv_fork_kernel<TX, TW, 4, V, 0><<<grid, 256, 0, st>>>(
         (const TX*)raw0, (const TX*)rawt, (const TW*)w, (const TW*)bias, (TX*)y0, (TX*)yt, (TX*)tails, L,
-        Cd, block, cold, kb0, cy);
+        Cd, block, cold, kb0, cy, seg);
   } else if (K == 4) {
     dim3 grid((cy + 255) / 256, nb, B);
     conv_fork_kernel<TX, TW, 4, 1, 0><<<grid, 256, 0, st>>>(
         (const TX*)raw0, (const TX*)rawt, (const TW*)w, (const TW*)bias, (TX*)y0, (TX*)yt, (TX*)tails, L,
-        Cd, block, cold, kb0, cy);
+        Cd, block, cold, kb0, cy, block);
   } else if (K == 2) {
     dim3 grid((cy + 255) / 256, nb, B);
     conv_fork_kernel<TX, TW, 2, 1, 0><<<grid, 256, 0, st>>>(
         (const TX*)raw0, (const TX*)rawt, (const TW*)w, (const TW*)bias, (TX*)y0, (TX*)yt, (TX*)tails, L,
-        Cd, block, cold, kb0, cy);
+        Cd, block, cold, kb0, cy, block);
   } else if (K == 3) {
     dim3 grid((cy + 255) / 256, nb, B);
     conv_fork_kernel<TX, TW, 3, 1, 0><<<grid, 256, 0, st>>>(
         (const TX*)raw0, (const TX*)rawt, (const TW*)w, (const TW*)bias, (TX*)y0, (TX*)yt, (TX*)tails, L,
-        Cd, block, cold, kb0, cy);
+        Cd, block, cold, kb0, cy, block);
   } else {
     return fail(DLLM_EUNSUPPORTED, "conv fork: kernel width %d not supported (2, 3 or 4)", K);
   }

@@ -162,3 +162,17 @@ def test_causal_conv1d_fn_package_keywords(dev):
         gdn.causal_conv1d_fn(x, w, seq_idx=torch.zeros(1, 20, dtype=torch.int32, device=dev))
     with pytest.raises(ValueError):
         gdn.causal_conv1d_fn(x, w, initial_states=pre, conv_prefix=pre)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("block", [32, 20, 12, 6, 3])
+@pytest.mark.parametrize("cold", [False, True])
+def test_fork_conv_rows_of_a_block_split(dev, dt, block, cold):
+    """A launch of few blocks cuts each block's rows in segments (of 4, 5, 3 rows, uncut at 3): the rows
+    after a cut see their own stream's rows before it, the block's first rows the clean prefix."""
+    raw0, rawt, w, b = _data(2, 3 * block, 72, 4, dt, dt, 900 + block, True)
+    got = _fork_conv(raw0, rawt, w, b, block, cold, dev)
+    ref = _fork_conv_ref(raw0, rawt, w, b, block, cold)
+    for name, g, r in zip(("y0", "yt"), got, ref):
+        _close(f"{name} block={block}", g, r, dt == torch.bfloat16)
+    assert torch.equal(got[2], ref[2])
