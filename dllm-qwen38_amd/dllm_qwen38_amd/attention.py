@@ -130,10 +130,15 @@ def _key_splits(q: torch.Tensor, M: int, N: int, Hkv: int, d: int) -> int:
     B * Hkv * ceil(rep / 4) workgroups or so: as many shares as fit one workgroup per CU (past it a
     second round costs more than shorter shares save: at B = 4, N = 4128, 24 / 4 heads of 256, 8
     shares 39.3 us, 16 53.0), of about four 32-key tiles each (fewer tiles save less than their
-    part of the merge costs: at B = 1, N = 2080, 12 to 20 shares 23.8-24.1 us, 8 25.5, 64 37.3). Up
-    to 160 keys one share is as fast (N = 160: 13.1 us, two shares 13.9)."""
+    part of the merge costs: at B = 1, N = 2080, 12 to 20 shares 23.8-24.1 us, 8 25.5, 64 37.3). One
+    share takes about 1 us per key tile, the split step 15 us and more with the rows that are merged: one
+    share up to 7 tiles of 256 (N = 224: 15.9 us, two shares 16.4; 320: 18.8, 16.4), 12 of 128 (384: 15.8, 16.1; 448:
+    17.4, 16.1) or 14 of 64 (448: 15.1, 16.1; 512: 16.6, 16.2), and one tile more per 2^17 merged values (24
+    heads of 256, B = 4: N = 384 20.8, 21.6; 512 24.4, 22.9; B = 16: N = 1024 42.1, 42.7; 1536 57.0, 50.3)."""
     tiles = -(-N // 32)
-    if q.dtype != torch.bfloat16 or d not in (64, 128, 256) or M > 64 or tiles <= 5:
+    if q.dtype != torch.bfloat16 or d not in (64, 128, 256) or M > 64:
+        return 1
+    if tiles <= {256: 7, 128: 12, 64: 14}[d] + (q.shape[0] * M * q.shape[2] * d >> 17):
         return 1
     B, rep = q.shape[0], q.shape[2] // Hkv
     hpw = 1 if rep == 1 else 4 if M <= 32 else 2 if rep % 2 == 0 else 1
