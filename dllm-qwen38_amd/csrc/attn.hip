@@ -77,6 +77,18 @@ __device__ __forceinline__ int attn_unit(int bid, int n, int chunk) {
   return ((i / chunk) * 8 + x) * chunk + i % chunk;
 }
 
+// Position in the longest-first order of dispatch slot bid among n, where every CU holds two workgroups of one
+// launch at once and n fills some CUs twice (256 < n <= 512): slot 256 + j joins slot j on its CU, so the longest units
+// take the CUs that stay with one, and the others are paired longest with shortest.
+// fp32 complementary mask, 24 / 4 heads of 256, B = 1, us without -> with: L = 256 (n = 384) 42.4 -> 32.4, L = 192 34.6 ->
+// 26.2, L = 320 58.5 -> 46.0; 16 / 4 heads of 128, L = 400 34.1 -> 27.5. (Counting a second workgroup's tiles from its last
+// wave: 33.3 at L = 256, 32.2 against 26.3 at L = 224.) A bijection of [0, n); the identity for other n.
+__device__ __forceinline__ int attn_pair_slot(int bid, int n) {
+  if (n <= 256 || n > 512) return bid;
+  const int r = n - 256;  // CUs with two
+  return bid < r ? 256 - r + bid : bid < 256 ? bid - r : n - 1 - (bid - 256);
+}
+
 // visibility of key block kb of half kh from query block qb of half qh (0 = x_t, 1 = x_0)
 __device__ __forceinline__ bool visible(int qh, int qb, int kh, int kb, int leak) {
   if (qh == 0) return kh == 0 ? (leak ? kb <= qb : kb == qb) : (kb < qb);
@@ -1054,7 +1066,7 @@ static int launch_attn_sp(const AttnArgs& a, hipStream_t st) {
 // operands come straight from L2 as fragments (K 16 bytes per lane, V^T 128 bytes per key and
 // instruction), a few slices ahead of their products, with no staging and no barrier in the loop; only Q
 // sits in LDS. Four 32-query tiles per workgroup with K/V staged for them, the kernel for the other layouts,
-// leaves most SIMDs idle at short lengths. B = 1, 24 / 4 heads of 256, us there -> here: L = 256 133 -> 42,
+// leaves most SIMDs idle at short lengths. B = 1, 24 / 4 heads of 256, us there -> here: L = 256 133 -> 42 (32 with attn_pair_slot),
 // L = 32 36 -> 15, L = 2048 1203 -> 1100 (103 TFLOP/s over the visible tiles); 32 rows of block-causal
 // queries against 4128 keys 1190 -> 284. Two slices ahead at D = 256: one 40 / 16 / 1023 / 388, three with
 // 512 registers a lane 42 / 16 / 954 / 275 (178 -> 189 at two sequences of 512).
@@ -1079,7 +1091,7 @@ __global__ __launch_bounds__(256, 2) void bd_attn_f32_kernel(AttnArgs a) {
 
   // work unit: longest first (query tile descending), then half, batch, KV head, query head in group
   constexpr int NH = BC ? 1 : 2;
-  const int lin = attn_unit(blockIdx.x, gridDim.x, NH * rep);
+  const int lin = attn_unit(attn_pair_slot(blockIdx.x, gridDim.x), gridDim.x, NH * rep);
   const int per_g = NH * a.B * a.Hkv * rep;
   const int r0 = (ntq - 1 - lin / per_g) * 32, r1 = min(Lq, r0 + 32);
   int rem = lin % per_g;

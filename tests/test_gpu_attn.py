@@ -151,3 +151,14 @@ def test_fp32_key_split_matches_oracle(dev, B, L, Hq, Hkv, d, block, leak, scale
     torch.cuda.synchronize()
     ref = attn_ref.bd_attention(q, k, v, block=block, scale=scale, leak_xt_prefix=leak)
     _check(got, ref, torch.float32, f"L{L} d{d} block{block} pad{pad}")
+
+
+@pytest.mark.parametrize("L", [264, 268, 508, 512, 520])
+def test_fp32_units_paired_on_a_cu(dev, L):
+    """Between 257 and 512 work units the dispatch order is permuted: every unit is still done once. Two halves of
+    ceil(L / 32) tiles and 16 heads: 288, 288, 512, 512 and 544 units."""
+    q, k, v = _inputs(1, L, 16, 4, 32, torch.float32, seed=L)
+    out = torch.full((1, 2 * L, 16, 32), float("nan"), device=dev)
+    got = attention.bd_attention(q.to(dev), k.to(dev), v.to(dev), block=4, out=out)
+    torch.cuda.synchronize()
+    _check(got, attn_ref.bd_attention(q, k, v, block=4), torch.float32, f"L{L}")
