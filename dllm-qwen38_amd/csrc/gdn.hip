@@ -1528,7 +1528,7 @@ extern "C" long long dllm_gdn_scan_workspace_bytes(int B, int T, int Hk, int Hv,
 
 // The fp32 fork by prepared tiles (gdn_scan_f32.hip): square heads of 64 or 128, blocks that divide the
 // 32-row tile, from one block on. Heads of 64 have a one-launch kernel, which takes over where a workgroup per
-// head fills the chip (L = 256: 128 heads 134 vs 95 us, 192 heads 139 vs 147; two blocks of four heads 36 vs 36).
+// head fills the chip (L = 256: 128 heads 128 vs 89 us, 192 heads 139 vs 147; two blocks of four heads 36 vs 36).
 extern "C" long long dllm_gdn_fork_f32_workspace_bytes(int B, int L, int Hk, int Hv, int Dk, int Dv, int block, int states) {
   if (B <= 0 || L <= 0 || Hk <= 0 || Hv <= 0 || block <= 0 || Hv % Hk || L % block || 32 % block) return 0;
   if (Dk != Dv || (Dk != 64 && Dk != 128)) return 0;

@@ -12,9 +12,9 @@
 // Bound by the fp32 matrix cores (about 12k clocks per SIMD at eight tiles of 48 heads of 128) and the state
 // chain (2.5k clocks a tile). The other path, the chunk kernel on the clean stream, then on every noised
 // block from its copied initial state, walked a tile's whole work in one chain and formed T twice per head:
-// conv and fork of one layer, 16 / 48 heads of 128, us there -> here: B = 1, L = 256 243 -> 87, L = 32 99 -> 39, B = 2,
-// L = 512 643 -> 268; four heads of 64, B = 1, L = 256 122 -> 47 (there one launch). The matrix cores are busy 44% of the
-// out and 36% of the prep kernel's time at L = 256, three waves a SIMD on them.
+// conv and fork of one layer, 16 / 48 heads of 128, us there -> here: B = 1, L = 256 243 -> 87, and 70 with the conv's rows
+// split (conv.hip), L = 32 99 -> 35, B = 2, L = 512 643 -> 252; four heads of 64, B = 1, L = 256 122 -> 38 (there one
+// launch). At L = 256 the kernels take 18, 20 and 25 us, the matrix cores busy 25, 32 and 38% of them.
 //
 // Workspace per (sequence, tile): per key head the clean K^T, per (head, stream) W and U (4 KB per 32 state rows / value columns each; the
 // state kernel leaves V' = U - W S of the clean stream in U's place), P (4 KB) and the row vectors; the
