@@ -9,7 +9,7 @@
 //                        on the fp32 matrix cores), not the 16 of a wave that also forms U, both outputs
 //                        and the update of all 128 rows;
 //   fork32_out_kernel    the outputs of every (tile, head, stream), a wave per 32 columns, no LDS.
-// Bound by the fp32 matrix cores (about 12k clocks per SIMD at eight tiles of 48 heads of 128) and the state
+// Bound by the fp32 matrix cores (40k clocks per SIMD in all at eight tiles of 48 heads of 128) and the state
 // chain (2.5k clocks a tile). The other path, the chunk kernel on the clean stream, then on every noised
 // block from its copied initial state, walked a tile's whole work in one chain and formed T twice per head:
 // conv and fork of one layer, 16 / 48 heads of 128, us there -> here: B = 1, L = 256 243 -> 87, and 70 with the conv's rows
